@@ -563,7 +563,7 @@ int openmini_qmm_gemm_f32(const openmini_qweight_t* weight, const float* d_x, fl
     if (rc != OPENMINI_QMM_OK) return rc;
     rc = check_f32_gemm_args(weight->w, d_x, d_y, m, d_work, work_bytes);
     if (rc != OPENMINI_QMM_OK) return rc;
-    hipError_t e = qmm::split_rows(d_x, m, weight->w.k, d_work, as_stream(stream));
+    hipError_t e = qmm::split_rows(weight->w, d_x, m, d_work, as_stream(stream));
     if (e == hipSuccess) e = qmm::launch_gemm_split(weight->w, d_work, m, d_y, as_stream(stream), false);
     if (e != hipSuccess) return hip_fail(e, "gemm_f32 launch");
     return ok();
@@ -654,7 +654,7 @@ int openmini_qmm_ffn_gate_up_f32(const openmini_qweight_t* gate, const openmini_
     rc = check_f32_gemm_args(gate->w, d_x, d_h, m, d_work, work_bytes);
     if (rc != OPENMINI_QMM_OK) return rc;
     // one split of x for both weights; the up GEMM finishes silu(gate) * up
-    hipError_t e = qmm::split_rows(d_x, m, gate->w.k, d_work, as_stream(stream));
+    hipError_t e = qmm::split_rows(gate->w, d_x, m, d_work, as_stream(stream));
     if (e == hipSuccess) e = qmm::launch_gemm_split(gate->w, d_work, m, d_h, as_stream(stream), false);
     if (e == hipSuccess) e = qmm::launch_gemm_split(up->w, d_work, m, d_h, as_stream(stream), true);
     if (e != hipSuccess) return hip_fail(e, "ffn_gate_up_f32 launch");
@@ -667,7 +667,7 @@ namespace {
 // workspace at d_work).
 hipError_t linear_rows(const qmm::Weight& w, const float* dx, float* dy, int64_t m, void* d_work) {
     if (gemm_rows(w, m)) {
-        hipError_t e = qmm::split_rows(dx, m, w.k, d_work, nullptr);
+        hipError_t e = qmm::split_rows(w, dx, m, d_work, nullptr);
         return e == hipSuccess ? qmm::launch_gemm_split(w, d_work, m, dy, nullptr, false) : e;
     }
     return qmm::launch_gemv_rows(w, nullptr, dx, dy, m, nullptr);

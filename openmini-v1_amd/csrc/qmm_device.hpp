@@ -70,4 +70,30 @@ __device__ __forceinline__ f16x8 codes_q8(uint32_t w0, uint32_t w1) {
     return __builtin_bit_cast(f16x8, *reinterpret_cast<uint4*>(p));
 }
 
+// Register transposes across the four 16-lane rows of a wave (gfx950 row swaps:
+// permlane32_swap exchanges rows 2, 3 of its first operand with rows 0, 1 of its
+// second; permlane16_swap rows 1, 3 of the first with rows 0, 2 of the second).
+// transpose4: register j of row r becomes register r of row j.
+__device__ __forceinline__ void transpose4(uint32_t& a0, uint32_t& a1, uint32_t& a2, uint32_t& a3) {
+    const auto p = __builtin_amdgcn_permlane32_swap(a0, a2, false, false);
+    const auto q = __builtin_amdgcn_permlane32_swap(a1, a3, false, false);
+    const auto u = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+    const auto v = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+    a0 = u[0];
+    a1 = u[1];
+    a2 = v[0];
+    a3 = v[1];
+}
+
+// broadcast4: out[t] holds row t of v in every row.
+__device__ __forceinline__ void broadcast4(float v, float* out) {
+    const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const auto a = __builtin_amdgcn_permlane32_swap(h[0], h[0], false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(h[1], h[1], false, false);
+    out[0] = __uint_as_float(a[0]);
+    out[1] = __uint_as_float(b[0]);
+    out[2] = __uint_as_float(a[1]);
+    out[3] = __uint_as_float(b[1]);
+}
+
 }  // namespace qmm

@@ -17,19 +17,31 @@
 // MFMA's 32, so q * scale (an exact integer of at most 13 bits) enters as bf16
 // hi + lo (two chained MFMAs, both exact), and the row's d is the block factor.
 //
-// Tiling: a workgroup computes a kBM x (16 kWT kNW) tile of y with kNW column slices
-// x kKS K parts of waves (choose_shape picks 128 or 64 rows and 3 or 2 weight tiles per
-// wave by problem size).  A wave owns kBM rows x 16 kWT columns (kBM/16 x kWT MFMA
+// Tiling: a workgroup of eight waves computes a kBM x (16 kWT kNW) tile of y with kNW
+// column slices x kKS K parts of waves (choose_shape picks one of six shapes, 128 x 192 to
+// 64 x 32, by problem size).  A wave owns kBM rows x 16 kWT columns (kBM/16 x kWT MFMA
 // subtiles of fp32 accumulators) over one K part, and the parts are added through
 // LDS at the end (fixed order).  A K step is two blocks (64 elements):
 //   * x: each K part's kBM x 64 bf16 slab is copied HBM -> LDS by buffer loads with
-//     an LDS destination (no registers), double-buffered, rows XOR-swizzled in
-//     16-byte segments so the A-fragment reads are bank-conflict free;
-//   * weights: each wave loads its kWT tiles' codes and scales straight into
-//     registers two K steps ahead (three register sets: first-touch weights come
-//     from HBM, whose latency under load exceeds one step) and converts its own B
-//     fragments (its columns are its own, so nothing is converted twice).
+//     an LDS destination (no registers) two steps ahead, rows XOR-swizzled in 16-byte
+//     segments so the A-fragment reads are bank-conflict free; the fragments of a half
+//     step are read while the half before it computes;
+//   * weights: each wave loads its kWT tiles' chunks straight into registers a group (4
+//     blocks) ahead, one wide load per tile, transposes them to the MFMA lanes by row
+//     swaps and converts its own B fragments (its columns are its own, so nothing is
+//     converted twice).
+// What bounds it: VALU issue.  Per half step and wave of the 128 x 192 shape, 24 MFMAs,
+// 96 rescale FMAs, 36 conversions and about 14 others are some 680 issue cycles, 51 us at
+// 512 rows of 11008 x 4096 and the 1.7 GHz the part holds under this load; with the copies,
+// weight loads and LDS reads it takes 65 us (from 72: until the stages were arrays of
+// their own, the compiler waited for every load just issued before each step's first
+// LDS read, so nothing was in flight across a step).  28672 x 8192 at 1024 rows: 638 ->
+// 575 us; few-row and fp32 shapes, where one workgroup has its CU alone and nothing else
+// hid those waits, gained most: Q8_0 4096 x 11008 at 100 fp32 rows 92 -> 40 us (with the
+// 64 x 32 shape, which fills the chip there).
 #include "qmm_device.hpp"
+
+#include <type_traits>
 
 namespace qmm {
 namespace {
@@ -85,20 +97,29 @@ struct GFmt {
     static constexpr int kScaleOff = kTileEntries * (kQ6K ? 24 : kCB);
     static constexpr int kDOff = kScaleOff + (kQ6K ? 2 : 1) * kTileEntries;  // K-quant: fp16 d per row
     static constexpr int kChunk = kQ4K ? kQ4KChunk : kQ6K ? kQ6KChunk : chunk_bytes_for(!kQ8);
-    // buffer loads one load_b issues per (tile, block), plus the K-quant d per tile
-    static constexpr int kLoadsPerBlock = kQ6K ? 3 : 2;
-    static constexpr int kLoadsPerTile = kKQ ? 1 : 0;
 };
 
-// A wave's weight operands for one K step: per weight tile j and block tt of the
-// step, the lane's 8 codes (Q4_0 / Q4_K one word of nibbles, Q8_0 two words of
-// bytes, Q6_K the low-nibble word and the top-bit word), its column's scale, and for
-// K-quants the column's d (one per step: a step stays inside one group).
-template <int kFmt, int kSB, int kWT>
-struct BRegs {
-    uint32_t c[kWT][kSB][GFmt<kFmt>::kWords];
-    uint32_t s[kWT][kSB];
-    uint32_t d[kWT];
+// A wave's weight operands for one group of 4 blocks, as loaded: per weight tile chunk
+// slot `lane` (block lane / 16, column lane % 16) whole -- its codes in one or two 16-byte
+// loads, its scale -- and for K-quants the column's d.  One wide load per tile and group
+// costs the address unit what one narrow load per block would.
+template <int kFmt, int kWT>
+struct BRaw {
+    uint4 c[kWT][GFmt<kFmt>::kQ8 ? 2 : 1];
+    uint2 h[GFmt<kFmt>::kQ6K ? kWT : 1];  // Q6_K: the slot's top code bits
+    uint32_t s[kWT];
+    uint32_t d[GFmt<kFmt>::kKQ ? kWT : 1];
+};
+
+// The same after the transpose across the wave's four 16-lane rows: for block t the
+// lane's 8 codes (elements 8 kq .. 8 kq + 7 of column li: Q4_0 / Q4_K one word of nibbles,
+// Q8_0 two words of bytes, Q6_K the low-nibble word and the top-bit word) and the block
+// factor (Q6_K: the column's scale pair as bits, its d in `d`).
+template <int kFmt, int kWT>
+struct BGroup {
+    uint32_t c[kWT][4][GFmt<kFmt>::kWords];
+    float f[kWT][4];
+    float d[GFmt<kFmt>::kQ6K ? kWT : 1];
 };
 
 // 8 Q6_K codes of lane quarter kq -> bf16 hi / lo parts of q * sc, q * sc exact (at
@@ -153,46 +174,59 @@ __device__ __forceinline__ void split_q6_f16(uint32_t w, uint32_t hm, int kq, fl
     lo = __builtin_bit_cast(f16x8, *reinterpret_cast<uint4*>(l));
 }
 
-// Workgroup shape: kBM x rows, kNW column slices x kKS K parts of waves; a K step is
-// kSB blocks.
-template <int kBM, int kNW, int kKS, int kSB, int kWT_>
+// Workgroup shape: kBM x rows, kNW column slices x kKS K parts of waves, two x stages in
+// LDS.  A step is one 128-byte piece of every x row: two blocks of bf16 x, one block of
+// split x (its hi and lo parts).
+template <int kBM, int kNW, int kKS, int kWT_>
 struct Shape {
     static constexpr int kWT = kWT_;                       // weight tiles (16 columns each) per wave
     static constexpr int kMI = kBM / 16;                   // MFMA row subtiles per wave
     static constexpr int kThreads = 64 * kNW * kKS;
     static constexpr int kBT = kNW * kWT;                 // weight tiles per workgroup
-    static constexpr int kRowB = kSB * kQK * 2;            // bytes of one x row per step
+    static constexpr int kRowB = 128;                      // bytes of one x row per step
     static constexpr int kSegs = kRowB / 16;               // 16-byte segments per row
     static constexpr int kSlabB = kBM * kRowB;             // one K part's x slab per step
     static constexpr int kStageB = kKS * kSlabB;
     static constexpr int kRowsPerCopy = 1024 / kRowB;      // one 1 KB copy instruction
     static constexpr int kCopies = kSlabB / kNW / 1024;     // copies per wave per step
-    static constexpr int kRedB = (kKS - 1) * kNW * kMI * kWT * 4 * 64 * 4;  // K-part partials
-    static constexpr int kLdsB = 2 * kStageB > kRedB ? 2 * kStageB : kRedB;
-    static_assert(kTileBlocks % kSB == 0, "a step covers whole blocks of one group");
+    static constexpr int kRedSlots = (kKS - 1) * kMI * kWT;  // K-part partials: 1 KB subtiles per column slice
+    // subtiles per column slice one stage array holds, and its bytes
+    static constexpr int kSlotsPerStage =
+        kStageB / 1024 / kNW > (kRedSlots + 1) / 2 ? kStageB / 1024 / kNW : (kRedSlots + 1) / 2;
+    static constexpr int kArrB = kSlotsPerStage * kNW * 1024;
+    static_assert(kCopies * kNW * 1024 == kSlabB, "whole copies per wave");
+    static_assert(kArrB >= kStageB, "a stage array holds a stage");
 };
 
-// kGate: y holds the gate projection on entry and each element is replaced by
+// Waves per SIMD the kernel is built for: two (one workgroup per CU, at most 256
+// registers).  The 64-row tiles of two weight tiles per wave come out at 115-130, and up to
+// 128 a CU runs two of them; Q8_0's 64 x 128 on bf16 x misses that by two, and held to it
+// runs 11008 x 4096 at 512 rows in 80 us instead of 91 (the other Q8_0 instances would
+// spill in the main loop: 64 x 64 40 -> 56 us at 100 rows of 4096 x 11008).
+template <int kFmt, int kBM, int kNW, int kWT, bool kX2>
+constexpr int kGemmWaves = kBM == 64 && kNW == 4 && kWT == 2 && kFmt == OPENMINI_QMM_Q8_0 && !kX2 ? 4 : 2;
+
+// gate_in_y: y holds the gate projection on entry and each element is replaced by
 // silu(gate) * (x . W^T), silu(v) = v / (1 + exp(-v)) (model.rs:713-735, :1187-1189).
-// kX2: x holds split fp32 activations (split_rows_kernel): per 32-element block 32 fp16
-// hi parts, then 32 fp16 lo parts, of x scaled by 2^e per row (x_exp[m] = e); k is
-// then the length of such a row in fp16 elements (twice K).  Each block runs two
-// chained fp16 MFMAs per subtile (hi, then lo, into one fp32 sum) with fp16 codes,
-// then the same rescale; outputs are scaled back by 2^-e.
-// Two waves per SIMD (512 / threads workgroups per CU): the register budget is 256.
-template <int kFmt, int kBM, int kNW, int kKS, int kSB, int kWT, bool kGate, bool kX2>
-__global__ __launch_bounds__(64 * kNW * kKS, 512 / (64 * kNW * kKS)) void gemm_kernel(
+// kX2: x holds split fp32 activations (split_rows_kernel), scaled by 2^e per row
+// (x_exp[m] = e).  Each block runs two chained fp16 MFMAs per subtile (hi, then lo, into
+// one fp32 sum) with fp16 codes, then the same rescale; outputs are scaled back by 2^-e.
+template <int kFmt, int kBM, int kNW, int kKS, int kWT, bool kX2>
+__global__ __launch_bounds__(64 * kNW * kKS, (kGemmWaves<kFmt, kBM, kNW, kWT, kX2>)) void gemm_kernel(
     const uint16_t* __restrict__ x, const int* __restrict__ x_exp, const uint8_t* __restrict__ chunks,
-    float* __restrict__ y, int m_rows, int n_rows, int n_tiles, int groups, int k) {
-    using S = Shape<kBM, kNW, kKS, kSB, kWT>;
+    float* __restrict__ y, int m_rows, int n_rows, int n_tiles, int groups, int k, int gate_in_y) {
+    using S = Shape<kBM, kNW, kKS, kWT>;
     using F = GFmt<kFmt>;
     constexpr int kMI = S::kMI;
-    constexpr int kCB = F::kCB;
     constexpr int kChunk = F::kChunk;
-    constexpr int kWB = kX2 ? kSB / 2 : kSB;  // weight blocks per step
-    static_assert(kWB >= 1, "a step holds at least one weight block");
-    constexpr int kStepsPerGroup = kTileBlocks / kWB;
-    __shared__ __attribute__((aligned(16))) uint8_t lds[S::kLdsB];
+    constexpr int kWB = kX2 ? 1 : 2;  // weight blocks per step
+    constexpr int kSPG = kTileBlocks / kWB;  // steps per group
+    // One array per x stage: the compiler then knows that a copy into one stage does not
+    // alias the fragment reads of another.  (With a single array it waited for every
+    // outstanding load before each step's first read, so nothing was in flight across
+    // a step.)
+    __shared__ __attribute__((aligned(16))) uint8_t lds0[S::kArrB];
+    __shared__ __attribute__((aligned(16))) uint8_t lds1[S::kArrB];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -203,69 +237,116 @@ __global__ __launch_bounds__(64 * kNW * kKS, 512 / (64 * kNW * kKS)) void gemm_k
     const int m0 = by * kBM;
     const int tile0 = bx * S::kBT + wn * kWT;
 
-    // this K part's steps; all parts step together (barriers), a shorter one idles
-    const int units = groups * kStepsPerGroup;
-    const int u0 = (int)((int64_t)units * kh / kKS);
-    const int u1 = (int)((int64_t)units * (kh + 1) / kKS);
-    const int steps = (units + kKS - 1) / kKS;
+    // this K part's groups; all parts step together (barriers), a shorter one idles
+    const int g0 = (int)((int64_t)groups * kh / kKS);
+    const int g1 = (int)((int64_t)groups * (kh + 1) / kKS);
+    const int g_last = max(g1 - 1, 0);
+    const int part_groups = (groups + kKS - 1) / kKS;
 
     // x is < 2 GiB (the launcher splits m); the chunks < 4 GiB (checked at upload)
-    const __amdgpu_buffer_rsrc_t x_rs = make_rsrc(x, (uint32_t)m_rows * (uint32_t)k * 2u);
+    const __amdgpu_buffer_rsrc_t x_rs = make_rsrc(x, (uint32_t)m_rows * (uint32_t)k * (kX2 ? 4u : 2u));
     const __amdgpu_buffer_rsrc_t w_rs = make_rsrc(chunks, (uint32_t)n_tiles * groups * kChunk);
 
-    // ---- x slab copies: kCopies x 1 KB per wave per step, kRowsPerCopy rows each.
-    // LDS position p of row r holds the row's 16-byte segment s = p ^ (r % kSegs).
-    // Offsets are recomputed per copy (registers are the scarce resource here).
+    // ---- x slab copies: kCopies x 1 KB per wave per step.
+    // bf16 x: kRowsPerCopy rows each; LDS position p of row r holds the row's 16-byte
+    // segment s = p ^ (r % kSegs), so the fragment reads are bank-conflict free.
+    // Split x: copy c is the hi (c even) or lo part of row subtile c / 2, which lies in
+    // memory as the MFMA reads it.
     const int r_lane = wn * (kBM / kNW) + lane / S::kSegs;
     const int p_lane = lane % S::kSegs;
-    auto issue_x = [&](int u, int stage) {
-        uint8_t* base = lds + stage * S::kStageB + kh * S::kSlabB + wn * S::kCopies * 1024;
-        const uint32_t kk0 = (uint32_t)u * (kSB * kQK);
+    const int nb = k / kQK;
+    const int x_tiles = (m_rows + 15) / 16;
+    auto issue_x = [&](int s, uint8_t* stage) {  // s: step of this part; past its end: zeros
+        const int g = g0 + s / kSPG, sub = s % kSPG;
+        const uint32_t k_lim = g < g1 ? (uint32_t)k : 0u;
+        uint8_t* base = stage + kh * S::kSlabB + wn * S::kCopies * 1024;
 #pragma unroll
         for (int j = 0; j < S::kCopies; ++j) {
-            const int r = r_lane + j * S::kRowsPerCopy;
-            const uint32_t seg = (uint32_t)((p_lane ^ (r % S::kSegs)) * 8) + kk0;
-            const uint32_t gm = (uint32_t)min(m0 + r, m_rows - 1);  // rows past m repeat the last one
-            // segments past K read zero (an out-of-range buffer offset)
-            const uint32_t voff = seg < (uint32_t)k ? (gm * (uint32_t)k + seg) * 2u : 0x80000000u;
+            uint32_t voff, soff = 0;
+            if constexpr (kX2) {
+                // a row tile is k / 32 pieces of 128 bytes per row; the last one may have
+                // fewer rows.  All offsets stay inside x: blocks past K repeat the last
+                // one (their weights are zero), tiles past m and rows past the tile
+                // repeat the last.
+                const int c = wn * S::kCopies + j;
+                const int rt = min(by * kMI + c / 2, x_tiles - 1);
+                const int rows = min(16, m_rows - rt * 16);
+                voff = (uint32_t)(kq * rows + min(li, rows - 1)) * 16u | (k_lim ? 0u : 0x80000000u);
+                soff = (uint32_t)rt * 64u * (uint32_t)k +
+                       (uint32_t)(min(min(g, g_last) * kTileBlocks + sub, nb - 1) * 2 + (c & 1)) * (uint32_t)rows * 64u;
+            } else {
+                const int r = r_lane + j * S::kRowsPerCopy;
+                const uint32_t seg = (uint32_t)((p_lane ^ (r % S::kSegs)) * 8) + (uint32_t)(g * kTileBlocks + sub * kWB) * kQK;
+                const uint32_t gm = (uint32_t)min(m0 + r, m_rows - 1);  // rows past m repeat the last one
+                // segments past K read zero (an out-of-range buffer offset)
+                voff = seg < k_lim ? (gm * (uint32_t)k + seg) * 2u : 0x80000000u;
+            }
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                x_rs, (__attribute__((address_space(3))) void*)(base + j * 1024), 16, voff, 0, 0, 0);
+                x_rs, (__attribute__((address_space(3))) void*)(base + j * 1024), 16, voff, soff, 0, 0);
         }
     };
 
-    // ---- weight operands: chunk (tile j, group g), slot (t, li), quarter kq
+    // ---- weight operands of one group
     uint32_t tile_off[kWT];
 #pragma unroll
     for (int j = 0; j < kWT; ++j) tile_off[j] = (uint32_t)min(tile0 + j, n_tiles - 1) * groups * kChunk;
-    auto load_b = [&](BRegs<kFmt, kWB, kWT>& B, int u) {
-        const int g = u / kStepsPerGroup, t0 = (u % kStepsPerGroup) * kWB;
+    auto load_b = [&](BRaw<kFmt, kWT>& R, int g) {
 #pragma unroll
         for (int j = 0; j < kWT; ++j) {
             const uint32_t soff = tile_off[j] + (uint32_t)g * kChunk;
-            if constexpr (F::kKQ) B.d[j] = __builtin_amdgcn_raw_buffer_load_b16(w_rs, F::kDOff + li * 2, soff, 0);
+            R.c[j][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(w_rs, lane * F::kCB, soff, 0));
+            if constexpr (F::kQ8)
+                R.c[j][1] =
+                    __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(w_rs, lane * F::kCB + 16, soff, 0));
+            if constexpr (F::kQ6K)
+                R.h[j] = __builtin_bit_cast(
+                    uint2, __builtin_amdgcn_raw_buffer_load_b64(w_rs, kTileEntries * 16 + lane * 8, soff, 0));
+            if constexpr (F::kQ4K)
+                R.s[j] = __builtin_amdgcn_raw_buffer_load_b8(w_rs, F::kScaleOff + lane, soff, 0);
+            else
+                R.s[j] = __builtin_amdgcn_raw_buffer_load_b16(w_rs, F::kScaleOff + lane * 2, soff, 0);
+            if constexpr (F::kKQ) R.d[j] = __builtin_amdgcn_raw_buffer_load_b16(w_rs, F::kDOff + li * 2, soff, 0);
+        }
+    };
+    // bf16 x runs Q4 codes as (q - 8) / 16: the block factor carries the 16 (exact)
+    constexpr float kUnit = F::kNib && !kX2 ? 16.0f : 1.0f;
+    auto unpack_b = [&](BGroup<kFmt, kWT>& B, const BRaw<kFmt, kWT>& R, bool live) {  // !live: factors 0
 #pragma unroll
-            for (int tt = 0; tt < kWB; ++tt) {
-                const uint32_t slot = (uint32_t)((t0 + tt) * kTileRows + li);
-                if constexpr (F::kQ4K)
-                    B.s[j][tt] = __builtin_amdgcn_raw_buffer_load_b8(w_rs, F::kScaleOff + slot, soff, 0);
-                else if constexpr (F::kQ6K)  // the scale of the lane's 16-element half
-                    B.s[j][tt] = __builtin_amdgcn_raw_buffer_load_b8(w_rs, F::kScaleOff + slot * 2 + (kq >> 1), soff, 0);
-                else
-                    B.s[j][tt] = __builtin_amdgcn_raw_buffer_load_b16(w_rs, F::kScaleOff + slot * 2, soff, 0);
-                if constexpr (F::kNib) {
-                    B.c[j][tt][0] = __builtin_amdgcn_raw_buffer_load_b32(w_rs, slot * kCB + kq * 4, soff, 0);
-                } else if constexpr (F::kQ6K) {
-                    B.c[j][tt][0] = __builtin_amdgcn_raw_buffer_load_b32(w_rs, slot * kCB + kq * 4, soff, 0);
-                    B.c[j][tt][1] = __builtin_amdgcn_raw_buffer_load_b32(
-                        w_rs, kTileEntries * 16 + slot * 8 + (kq >> 1) * 4, soff, 0);
-                } else {
-                    const uint2 v = __builtin_bit_cast(
-                        uint2, __builtin_amdgcn_raw_buffer_load_b64(w_rs, slot * kCB + kq * 8, soff, 0));
-                    B.c[j][tt][0] = v.x;
-                    B.c[j][tt][1] = v.y;
+        for (int j = 0; j < kWT; ++j) {
+            uint32_t e[4], o[4];
+            const uint4 c = R.c[j][0];
+            if constexpr (F::kQ8) {
+                const uint4 c1 = R.c[j][1];
+                e[0] = c.x; o[0] = c.y; e[1] = c.z; o[1] = c.w;
+                e[2] = c1.x; o[2] = c1.y; e[3] = c1.z; o[3] = c1.w;
+                transpose4(e[0], e[1], e[2], e[3]);
+                transpose4(o[0], o[1], o[2], o[3]);
+            } else {
+                e[0] = c.x; e[1] = c.y; e[2] = c.z; e[3] = c.w;
+                transpose4(e[0], e[1], e[2], e[3]);
+                if constexpr (F::kQ6K) {  // lane (kq, i) takes top-bit word kq / 2
+                    o[0] = R.h[j].x; o[1] = R.h[j].x; o[2] = R.h[j].y; o[3] = R.h[j].y;
+                    transpose4(o[0], o[1], o[2], o[3]);
                 }
             }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                B.c[j][t][0] = e[t];
+                if constexpr (F::kWords == 2) B.c[j][t][1] = o[t];
+            }
+            if constexpr (F::kQ6K) {
+                broadcast4(__uint_as_float(R.s[j]), B.f[j]);
+                B.d[j] = live ? f16_bits_to_f32((uint16_t)R.d[j]) : 0.0f;
+            } else if constexpr (F::kQ4K) {
+                broadcast4(live ? f16_bits_to_f32((uint16_t)R.d[j]) * (float)(R.s[j] & 0xFFu) * kUnit : 0.0f, B.f[j]);
+            } else {
+                broadcast4(live ? f16_bits_to_f32((uint16_t)R.s[j]) * kUnit : 0.0f, B.f[j]);
+            }
         }
+    };
+    // Q6_K: a quarter of the scale of the lane's 16-element half of block t (exact)
+    auto q6_scale = [&](const BGroup<kFmt, kWT>& B, int j, int t) {
+        return (float)(int8_t)((__float_as_uint(B.f[j][t]) >> ((kq >> 1) * 8)) & 0xFFu) * 0.25f;
     };
 
     f32x4 acc[kMI][kWT];
@@ -278,32 +359,35 @@ __global__ __launch_bounds__(64 * kNW * kKS, 512 / (64 * kNW * kKS)) void gemm_k
 #pragma unroll
         for (int j = 0; j < kWT; ++j) acc[i][j] = sacc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // A fragments of 32-element segment tt of the step in LDS stage `stage`: rows
-    // i * 16 + li, elements 8 kq .. 8 kq + 7 of the segment (swizzled); bf16 x, or the
-    // fp16 hi (tt even) / lo (tt odd) parts of one block of split x.
+    // A fragments of half h of the step in `stage`: rows i * 16 + li, elements 8 kq ..
+    // 8 kq + 7 of bf16 block h; or of split x's row subtiles h kMI / 2 + i / 2 the fp16 hi
+    // (i even) / lo (i odd) parts.
     typedef uint4 AFrags[kMI];
-    auto read_a = [&](AFrags& a, int stage, int tt) {
-        const uint8_t* slab = lds + stage * S::kStageB + kh * S::kSlabB;
+    auto read_a = [&](AFrags& a, const uint8_t* stage, int h) {
+        const uint8_t* slab = stage + kh * S::kSlabB;
 #pragma unroll
         for (int i = 0; i < kMI; ++i) {
-            const int r = i * 16 + li;
-            a[i] = *reinterpret_cast<const uint4*>(slab + r * S::kRowB + (((tt * 4 + kq) ^ (r % S::kSegs)) * 16));
+            if constexpr (kX2) {
+                a[i] = *reinterpret_cast<const uint4*>(slab + (h * kMI + i) * 1024 + lane * 16);
+            } else {
+                const int r = i * 16 + li;
+                a[i] = *reinterpret_cast<const uint4*>(slab + r * S::kRowB + (((h * 4 + kq) ^ (r % S::kSegs)) * 16));
+            }
         }
     };
     auto bf = [](const uint4& v) { return __builtin_bit_cast(bf16x8, v); };
     auto hf = [](const uint4& v) { return __builtin_bit_cast(f16x8, v); };
-    // Q6_K block tt: the scale changes every 16 elements, inside an MFMA's 32, so it is
-    // folded into the codes: q * sc (exact integers) as bf16 hi + lo.  The d is one per
+    // Q6_K block t: the scale changes every 16 elements, inside an MFMA's 32, so it
+    // is folded into the codes: q * sc (exact integers) as bf16 hi + lo.  The d is one per
     // tile row and super-block, so the blocks of a super-block chain into one sum per
     // output (sacc; all hi MFMAs, then all lo ones, so no MFMA waits on the one before),
     // and flush_q6 applies d once per super-block: one FMA per output per 8 blocks
     // instead of one per block.
-    auto compute_q6 = [&](const BRegs<kFmt, kWB, kWT>& B, const AFrags& a, int tt) {
-        if constexpr (F::kQ6K && !kX2) {
+    auto compute_q6 = [&](const BGroup<kFmt, kWT>& B, const AFrags& a, int t) {
+        if constexpr (kChain) {
             bf16x8 bh[kWT], bl[kWT];
 #pragma unroll
-            for (int j = 0; j < kWT; ++j)
-                split_q6(B.c[j][tt][0], B.c[j][tt][1], kq, (float)(int8_t)(B.s[j][tt] & 0xFFu) * 0.25f, bh[j], bl[j]);
+            for (int j = 0; j < kWT; ++j) split_q6(B.c[j][t][0], B.c[j][t][1], kq, q6_scale(B, j, t), bh[j], bl[j]);
 #pragma unroll
             for (int q = 0; q < kMI * kWT; ++q)
                 sacc[q / kWT][q % kWT] =
@@ -314,42 +398,32 @@ __global__ __launch_bounds__(64 * kNW * kKS, 512 / (64 * kNW * kKS)) void gemm_k
                     __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf(a[q / kWT]), bl[q % kWT], sacc[q / kWT][q % kWT], 0, 0, 0);
         }
     };
-    // Q6_K: after the last block of a super-block, or of this K part, acc += sacc * d.
-    auto flush_q6 = [&](const BRegs<kFmt, kWB, kWT>& B) {
+    // Q6_K: after the last group of a super-block, or of this K part, acc += sacc * d.
+    auto flush_q6 = [&](const BGroup<kFmt, kWT>& B) {
         if constexpr (kChain) {
 #pragma unroll
-            for (int j = 0; j < kWT; ++j) {
-                const float d = f16_bits_to_f32((uint16_t)B.d[j]);
+            for (int j = 0; j < kWT; ++j)
 #pragma unroll
                 for (int i = 0; i < kMI; ++i) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(sacc[i][j][r], d, acc[i][j][r]);
+                    for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(sacc[i][j][r], B.d[j], acc[i][j][r]);
                     sacc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
-            }
         }
     };
-    // Block tt of one step: 8 x 3 MFMAs on A fragments `a` and the weight registers.
-    auto compute = [&](const BRegs<kFmt, kWB, kWT>& B, const AFrags& a, int tt) {
+    // Block t of the group on bf16 fragments `a`: kMI x kWT MFMAs and their rescales.
+    auto compute = [&](const BGroup<kFmt, kWT>& B, const AFrags& a, int t) {
         if constexpr (F::kQ6K) {
-            compute_q6(B, a, tt);
+            compute_q6(B, a, t);
             return;
         }
         bf16x8 b[kWT];
-        float d[kWT];
 #pragma unroll
         for (int j = 0; j < kWT; ++j) {
-            const uint16_t dh = (uint16_t)B.s[j][tt];
-            if constexpr (F::kQ4K) {  // (q - 8) / 16 codes; block factor 16 d * scale (exact)
-                b[j] = cvt_q4(B.c[j][tt][0]);
-                d[j] = f16_bits_to_f32((uint16_t)B.d[j]) * (float)(B.s[j][tt] & 0xFFu) * 16.0f;
-            } else if constexpr (F::kNib) {
-                b[j] = cvt_q4(B.c[j][tt][0]);
-                d[j] = f16_bits_to_f32(dh) * 16.0f;
-            } else {
-                b[j] = cvt_q8(B.c[j][tt][0], B.c[j][tt][1]);
-                d[j] = f16_bits_to_f32(dh);
-            }
+            if constexpr (F::kNib)
+                b[j] = cvt_q4(B.c[j][t][0]);
+            else
+                b[j] = cvt_q8(B.c[j][t][0], B.c[j][t][1]);
         }
         // MFMA q + 1 is issued before the FMAs of q (two result registers)
         f32x4 pp[2];
@@ -361,139 +435,139 @@ __global__ __launch_bounds__(64 * kNW * kKS, 512 / (64 * kNW * kKS)) void gemm_k
                     bf(a[(q + 1) / kWT]), b[(q + 1) % kWT], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                acc[q / kWT][q % kWT][r] = fmaf(pp[q & 1][r], d[q % kWT], acc[q / kWT][q % kWT][r]);
+                acc[q / kWT][q % kWT][r] = fmaf(pp[q & 1][r], B.f[q % kWT][t], acc[q / kWT][q % kWT][r]);
         }
     };
-    // Split x, the step's one block: per subtile the hi and the lo fragments times the
-    // same fp16 codes, chained into one fp32 sum (exact products), then the rescale.
-    // Q6_K: q * scale as fp16 hi + lo codes, four chained MFMAs per subtile.  (Chaining
-    // a super-block's blocks as on bf16 x was slower here: 194 -> 225 us at M = 512;
-    // these four MFMAs per block outweigh the rescale, and the chained sums' registers
-    // rule out the 128 x 96 tiles.)
-    auto compute_x2 = [&](const BRegs<kFmt, kWB, kWT>& B, const AFrags& ah, const AFrags& al) {
-        if constexpr (kX2) {
-            constexpr int kCodes = F::kQ6K ? 2 : 1;
-            f16x8 b[kWT][kCodes];
-            float d[kWT];
+    // Split x, block t, half h of its row subtiles: per subtile the hi and the lo
+    // fragments times the same fp16 codes, chained into one fp32 sum (exact products),
+    // then the rescale.  Q6_K: q * scale as fp16 hi + lo codes, four chained MFMAs per
+    // subtile.  (Chaining a super-block's blocks as on bf16 x was slower here: 194 -> 225
+    // us at M = 512; these four MFMAs per block outweigh the rescale, and the chained
+    // sums' registers rule out the wide tiles.)
+    constexpr int kCodes = F::kQ6K ? 2 : 1;
+    typedef f16x8 BX2[kWT][kCodes];
+    auto convert_x2 = [&](BX2& b, const BGroup<kFmt, kWT>& B, int t) {
 #pragma unroll
-            for (int j = 0; j < kWT; ++j) {
-                if constexpr (F::kQ6K) {
-                    split_q6_f16(B.c[j][0][0], B.c[j][0][1], kq, (float)(int8_t)(B.s[j][0] & 0xFFu) * 0.25f, b[j][0],
-                                 b[j][1]);
-                    d[j] = f16_bits_to_f32((uint16_t)B.d[j]);
-                } else if constexpr (F::kQ4K) {  // q - 8 codes; block factor d * scale (exact)
-                    b[j][0] = codes_q4(B.c[j][0][0]);
-                    d[j] = f16_bits_to_f32((uint16_t)B.d[j]) * (float)(B.s[j][0] & 0xFFu);
-                } else if constexpr (F::kNib) {
-                    b[j][0] = codes_q4(B.c[j][0][0]);
-                    d[j] = f16_bits_to_f32((uint16_t)B.s[j][0]);
-                } else {
-                    b[j][0] = codes_q8(B.c[j][0][0], B.c[j][0][1]);
-                    d[j] = f16_bits_to_f32((uint16_t)B.s[j][0]);
-                }
+        for (int j = 0; j < kWT; ++j) {
+            if constexpr (F::kQ6K)
+                split_q6_f16(B.c[j][t][0], B.c[j][t][1], kq, q6_scale(B, j, t), b[j][0], b[j][kCodes - 1]);
+            else if constexpr (F::kNib)
+                b[j][0] = codes_q4_perm(B.c[j][t][0]);  // split x is stored in its order
+            else
+                b[j][0] = codes_q8(B.c[j][t][0], B.c[j][t][F::kWords - 1]);
+        }
+    };
+    auto compute_x2 = [&](const BX2& b, const BGroup<kFmt, kWT>& B, const AFrags& a, int t, int h) {
+        constexpr int kHalf = kMI / 2;
+        auto block = [&](int q) {
+            const int i = q / kWT, j = q % kWT;
+            f32x4 v = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf(a[2 * i]), b[j][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            v = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf(a[2 * i + 1]), b[j][0], v, 0, 0, 0);
+#pragma unroll
+            for (int c = 1; c < kCodes; ++c) {
+                v = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf(a[2 * i]), b[j][c], v, 0, 0, 0);
+                v = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf(a[2 * i + 1]), b[j][c], v, 0, 0, 0);
             }
-            auto block = [&](int q) {
-                const int i = q / kWT, j = q % kWT;
-                f32x4 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf(ah[i]), b[j][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf(al[i]), b[j][0], t, 0, 0, 0);
+            return v;
+        };
+        // the MFMAs of subtile q + 1 are issued before the FMAs of q
+        f32x4 pp[2];
+        pp[0] = block(0);
 #pragma unroll
-                for (int c = 1; c < kCodes; ++c) {
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf(ah[i]), b[j][c], t, 0, 0, 0);
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(hf(al[i]), b[j][c], t, 0, 0, 0);
-                }
-                return t;
-            };
-            // the MFMAs of subtile q + 1 are issued before the FMAs of q
-            f32x4 pp[2];
-            pp[0] = block(0);
+        for (int q = 0; q < kHalf * kWT; ++q) {
+            if (q + 1 < kHalf * kWT) pp[(q + 1) & 1] = block(q + 1);
+            const int i = h * kHalf + q / kWT, j = q % kWT;
+            float d;
+            if constexpr (F::kQ6K) d = B.d[j]; else d = B.f[j][t];
 #pragma unroll
-            for (int q = 0; q < kMI * kWT; ++q) {
-                if (q + 1 < kMI * kWT) pp[(q + 1) & 1] = block(q + 1);
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    acc[q / kWT][q % kWT][r] = fmaf(pp[q & 1][r], d[q % kWT], acc[q / kWT][q % kWT][r]);
-            }
+            for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(pp[q & 1][r], d, acc[i][j][r]);
         }
     };
 
-    // Step `it` (unit u = u0 + it): the x copies for u were issued one step earlier,
-    // the weights for u two steps earlier.  Per step the wave issues x(u + 1), then
-    // the weights of u + 2 (kBLoads loads), so waiting until at most kBLoads loads
-    // are outstanding completes x(u) and everything older; one barrier then makes
-    // every wave's copies visible and frees the other x stage.  The loads are
-    // unconditional (units past this part's end re-load its last unit, a cache hit)
-    // so the count of outstanding loads is the same on every path; the compiler's
-    // own waits before the barrier then cover only the x copies.
-    constexpr int kBLoads = kWT * (kWB * F::kLoadsPerBlock + F::kLoadsPerTile);
+    // Step s runs as two halves, each with the fragments of the next half on their way
+    // from LDS.  Between the halves the wave waits for x(s + 1) -- until at most the loads
+    // issued after its copies are outstanding -- and for its own fragment reads of
+    // step s; one barrier then makes every wave's copies visible and frees the stage of
+    // step s, which takes x(s + 2).  A group's first step loads the next group's
+    // weights, after its first half (issued right after the copies, every wave of the
+    // CU would queue its vector-memory instructions at once and stall its MFMAs behind
+    // them).  The loads are unconditional (steps past this part's end repeat its last
+    // group, cache hits), so the count of outstanding loads is the same on every path; the
+    // memory clobbers keep their order.  With one column slice every wave reads only
+    // what it copied itself, and no barrier is needed.
+    // A half's MFMAs and rescale run at raised wave priority, so the SIMD's other wave
+    // yields issue slots to them.
+    constexpr int kBLoads = kWT * ((F::kQ8 || F::kQ6K ? 3 : 2) + (F::kKQ ? 1 : 0));
     static_assert(kBLoads <= 63, "vmcnt counts up to 63");
-    const int u_last = max(u1 - 1, 0);
-    // Q6_K: unit u holds blocks u kWB .. u kWB + kWB - 1 of the row; a super-block is 8
-    // blocks, and a K part may start or end inside one
-    auto q6_ends = [&](int u) { return kChain && (((u + 1) * kWB) % 8 == 0 || u == u1 - 1); };
-    auto step = [&](int it, const BRegs<kFmt, kWB, kWT>& cur, BRegs<kFmt, kWB, kWT>& far) {
-        const int u = u0 + it;
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(kBLoads));
-        __syncthreads();
-        issue_x(min(u + 1, u_last), (it + 1) & 1);
-        // The weight loads go between the step's blocks: issued right after the copies,
-        // every wave of the CU would queue its vector-memory instructions at once and
-        // stall its MFMAs behind them.  The memory clobbers keep the issue order (the
-        // copies before the weights) that the vmcnt count above relies on.
+    // Q6_K's 128-row tiles have no registers for a second set: they read each half's
+    // fragments just before it (the second half's before the wait, its stage being
+    // overwritten after it).
+    constexpr bool kAhead = !(F::kQ6K && kBM == 128);
+    AFrags f0, f1;
+    // Keeps memory operations in order, and the scheduler from moving one half's work (the
+    // next blocks' code conversions above all) into another, which would not fit the
+    // registers.
+    auto fence = [] {
         asm volatile("" ::: "memory");
-        const bool live = u < u1;  // uniform per wave
-        if constexpr (kX2) {  // one block per step: its hi and lo fragments, then the weights
-            AFrags ah, al;
-            if (live) {
-                read_a(ah, it & 1, 0);
-                read_a(al, it & 1, 1);
-                __builtin_amdgcn_s_setprio(3);
-                compute_x2(cur, ah, al);
-                __builtin_amdgcn_s_setprio(0);
-            }
-            asm volatile("" ::: "memory");
-            load_b(far, min(u + 2, u_last));
-            asm volatile("" ::: "memory");
-            if (live && q6_ends(u)) flush_q6(cur);
-            return;
-        }
-        AFrags a;
-        // A block's MFMAs and rescale run at raised wave priority, so the SIMD's other
-        // wave (copies, weight loads, a barrier) yields issue slots to them: Q8_0
-        // M=512 83.5-83.7 -> 81.9-82.1 us, Q4_0 28672x8192 M=1024 598-601 -> 588-591 us
-        // (three interleaved passes, one box; priority 1 gained about half of that).
-        if (live) {
-            read_a(a, it & 1, 0);
-            __builtin_amdgcn_s_setprio(3);
-            compute(cur, a, 0);
-            __builtin_amdgcn_s_setprio(0);
-        }
-        asm volatile("" ::: "memory");
-        load_b(far, min(u + 2, u_last));
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int tt = 1; tt < kSB; ++tt)
-            if (live) {
-                read_a(a, it & 1, tt);
-                __builtin_amdgcn_s_setprio(3);
-                compute(cur, a, tt);
-                __builtin_amdgcn_s_setprio(0);
-            }
-        if (live && q6_ends(u)) flush_q6(cur);
+        __builtin_amdgcn_sched_barrier(0);
     };
-
-    BRegs<kFmt, kWB, kWT> b0, b1, b2;
-    issue_x(min(u0, u_last), 0);
+    auto step = [&](int gi, int sub, const BGroup<kFmt, kWT>& B, BRaw<kFmt, kWT>& next, uint8_t* now,
+                    const uint8_t* after) {
+        const int s = gi * kSPG + sub;
+        BX2 bx;
+        if constexpr (kAhead) read_a(f1, now, 1);
+        else read_a(f0, now, 0);
+        fence();
+        __builtin_amdgcn_s_setprio(3);
+        if constexpr (kX2) {
+            convert_x2(bx, B, sub);
+            compute_x2(bx, B, f0, sub, 0);
+        } else {
+            compute(B, f0, sub * 2);
+        }
+        __builtin_amdgcn_s_setprio(0);
+        fence();
+        if (sub == 0) load_b(next, min(g0 + gi + 1, g_last));
+        if constexpr (!kAhead) read_a(f0, now, 1);
+        fence();
+        if (sub == 0)  // constant after unrolling
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(kBLoads) & ~0x0F00);
+        else
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(0) & ~0x0F00);
+        if constexpr (kNW > 1) __builtin_amdgcn_s_barrier();
+        fence();
+        issue_x(s + 2, now);
+        fence();
+        if constexpr (kAhead) read_a(f0, after, 0);
+        fence();
+        __builtin_amdgcn_s_setprio(3);
+        if constexpr (kX2)
+            compute_x2(bx, B, kAhead ? f1 : f0, sub, 1);
+        else
+            compute(B, kAhead ? f1 : f0, sub * 2 + 1);
+        __builtin_amdgcn_s_setprio(0);
+        const int g = g0 + gi;
+        if (sub == kSPG - 1 && kChain && ((g & 1) == 1 || g >= g1 - 1)) flush_q6(B);
+    };
+    issue_x(0, lds0);
+    issue_x(1, lds1);
+    BRaw<kFmt, kWT> raw;
+    load_b(raw, min(g0, g_last));
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+    if constexpr (kNW > 1) __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    load_b(b0, min(u0, u_last));
-    load_b(b1, min(u0 + 1, u_last));
-    int it = 0;
-    for (; it + 2 < steps; it += 3) {  // three register sets rotate: no copies
-        step(it, b0, b2);
-        step(it + 1, b1, b0);
-        step(it + 2, b2, b1);
+    if constexpr (kAhead) read_a(f0, lds0, 0);
+    BGroup<kFmt, kWT> B;
+    unpack_b(B, raw, g0 < g1);
+    for (int gi = 0; gi < part_groups; ++gi) {
+        step(gi, 0, B, raw, lds0, lds1);
+        step(gi, 1, B, raw, lds1, lds0);
+        if constexpr (kSPG == 4) {
+            step(gi, 2, B, raw, lds0, lds1);
+            step(gi, 3, B, raw, lds1, lds0);
+        }
+        unpack_b(B, raw, g0 + gi + 1 < g1);
     }
-    if (it < steps) step(it, b0, b2);
-    if (it + 1 < steps) step(it + 1, b1, b0);
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // no copy may land after the stages are reused
 
     // ---- K parts meet in LDS (the stages are free after this barrier), then store.
@@ -501,23 +575,29 @@ __global__ __launch_bounds__(64 * kNW * kKS, 512 / (64 * kNW * kKS)) void gemm_k
     // part 0 issues all its LDS reads together, adds the parts in order (fixed, so the
     // bits do not depend on timing) and stores.
     __syncthreads();
-    f32x4* red = reinterpret_cast<f32x4*>(lds);
-    auto slot = [&](int h, int i, int j) { return ((((h - 1) * kNW + wn) * kMI + i) * kWT + j) * 64 + lane; };
-    if (kh > 0) {
+    auto slot = [&](int h, int i, int j) {
+        const int l = (h - 1) * kMI * kWT + i * kWT + j, arr = l / S::kSlotsPerStage;
+        uint8_t* base = arr == 0 ? lds0 : lds1;
+        return reinterpret_cast<f32x4*>(base) + ((l % S::kSlotsPerStage) * kNW + wn) * 64 + lane;
+    };
 #pragma unroll
-        for (int i = 0; i < kMI; ++i)
+    for (int h = 1; h < kKS; ++h)
+        if (kh == h) {
 #pragma unroll
-            for (int j = 0; j < kWT; ++j) red[slot(kh, i, j)] = acc[i][j];
-    }
+            for (int i = 0; i < kMI; ++i)
+#pragma unroll
+                for (int j = 0; j < kWT; ++j) *slot(h, i, j) = acc[i][j];
+        }
     __syncthreads();
     if (kh == 0) {
 #pragma unroll
         for (int h = 1; h < kKS; ++h) {
+            fence();
             f32x4 part[kMI][kWT];  // all of a part's reads in flight before the first add
 #pragma unroll
             for (int i = 0; i < kMI; ++i)
 #pragma unroll
-                for (int j = 0; j < kWT; ++j) part[i][j] = red[slot(h, i, j)];
+                for (int j = 0; j < kWT; ++j) part[i][j] = *slot(h, i, j);
 #pragma unroll
             for (int i = 0; i < kMI; ++i)
 #pragma unroll
@@ -531,88 +611,96 @@ __global__ __launch_bounds__(64 * kNW * kKS, 512 / (64 * kNW * kKS)) void gemm_k
 #pragma unroll
                 for (int r = 0; r < 4; ++r) rexp[i][r] = -x_exp[min(m0 + i * 16 + kq * 4 + r, m_rows - 1)];
         }
-        // lane holds D[4 kq + r][li] of each 16 x 16 subtile
-        auto store = [&](int i, int j, int r) {
-            float* yp = y + (size_t)(m0 + i * 16 + kq * 4 + r) * n_rows + (tile0 + j) * kTileRows + li;
-            float v = acc[i][j][r];
-            if constexpr (kX2) v = __builtin_amdgcn_ldexpf(v, rexp[i][r]);
-            if constexpr (kGate) {
-                const float g = *yp;
-                v = g / (1.0f + expf(-g)) * v;
-            }
-            *yp = v;
-        };
-        if (m0 + kBM <= m_rows && (tile0 + kWT) * kTileRows <= n_rows) {  // whole tile inside y
+        // lane holds D[4 kq + r][li] of each 16 x 16 subtile; a row subtile's gate values
+        // are read together, before its first store
+        auto put = [&](int j, auto gated, auto inside) {
 #pragma unroll
-            for (int j = 0; j < kWT; ++j)
-#pragma unroll
-                for (int i = 0; i < kMI; ++i)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) store(i, j, r);
-        } else {
-#pragma unroll
-            for (int j = 0; j < kWT; ++j)
-#pragma unroll
-                for (int i = 0; i < kMI; ++i)
+            for (int i = 0; i < kMI; ++i) {
+                float* yp = y + (size_t)(m0 + i * 16 + kq * 4) * n_rows + (tile0 + j) * kTileRows + li;
+                float gate[4] = {0.f, 0.f, 0.f, 0.f};
+                if constexpr (gated) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        if (m0 + i * 16 + kq * 4 + r < m_rows && (tile0 + j) * kTileRows + li < n_rows) store(i, j, r);
+                        if (inside(i, j, r)) gate[r] = yp[(size_t)r * n_rows];
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float v = acc[i][j][r];
+                    if constexpr (kX2) v = __builtin_amdgcn_ldexpf(v, rexp[i][r]);
+                    if constexpr (gated) v = gate[r] / (1.0f + expf(-gate[r])) * v;
+                    if (inside(i, j, r)) yp[(size_t)r * n_rows] = v;
+                }
+            }
+        };
+        auto all = [](int, int, int) { return true; };
+        auto some = [&](int i, int j, int r) {
+            return m0 + i * 16 + kq * 4 + r < m_rows && (tile0 + j) * kTileRows + li < n_rows;
+        };
+        if (m0 + kBM <= m_rows && (tile0 + kWT) * kTileRows <= n_rows && !gate_in_y) {  // whole tile inside y
+#pragma unroll
+            for (int j = 0; j < kWT; ++j) put(j, std::false_type{}, all);
+        } else if (!gate_in_y) {
+#pragma unroll
+            for (int j = 0; j < kWT; ++j) put(j, std::false_type{}, some);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kWT; ++j) put(j, std::true_type{}, some);
         }
     }
 }
 
-// x rows of kx 2-byte elements (K for bf16 x, 2 K for split x).
-template <int kFmt, int kBM, int kNW, int kKS, int kSB, int kWT, bool kGate, bool kX2>
-hipError_t launch_shape(const Weight& w, const uint16_t* x, const int* x_exp, float* y, int64_t m, int64_t kx,
+// x rows of k elements (bf16, or split fp32: 4 bytes per element).
+template <int kFmt, int kBM, int kNW, int kKS, int kWT, bool kX2>
+hipError_t launch_shape(const Weight& w, const uint16_t* x, const int* x_exp, float* y, int64_t m, bool gate_in_y,
                         hipStream_t s) {
-    using S = Shape<kBM, kNW, kKS, kSB, kWT>;
+    using S = Shape<kBM, kNW, kKS, kWT>;
     const dim3 grid((unsigned)((w.n_tiles + S::kBT - 1) / S::kBT), (unsigned)((m + kBM - 1) / kBM));
-    hipLaunchKernelGGL((gemm_kernel<kFmt, kBM, kNW, kKS, kSB, kWT, kGate, kX2>), grid, dim3(S::kThreads), 0, s, x,
-                       x_exp, w.chunks, y, (int)m, (int)w.n, (int)w.n_tiles, (int)w.groups, (int)kx);
+    hipLaunchKernelGGL((gemm_kernel<kFmt, kBM, kNW, kKS, kWT, kX2>), grid, dim3(S::kThreads), 0, s, x, x_exp, w.chunks,
+                       y, (int)m, (int)w.n, (int)w.n_tiles, (int)w.groups, (int)w.k, (int)gate_in_y);
     return hipGetLastError();
 }
 
-// Tile families: 128-row tiles with 2 column slices x 2 K halves of waves (64 KB of LDS,
-// two workgroups per CU so one's barriers overlap the other's work), and 64-row tiles
-// with 2 column slices x 4 K parts (72 KB of LDS) for more, smaller workgroups.  Split
-// x uses the same shapes with one block per step (its hi and lo parts fill the step's
-// 64-element slab).
-// Launch shape by problem size.
-//   0: 128-row tiles, 3 weight tiles per wave (128 x 96, 4 waves)
-//   1: 128-row tiles, 2 weight tiles per wave (128 x 64, 4 waves)
-//   2:  64-row tiles, 3 weight tiles per wave ( 64 x 96, 8 waves)
-//   3:  64-row tiles, 2 weight tiles per wave ( 64 x 64, 8 waves)
-// Few and large workgroups leave CUs idle or a last round part-filled; small ones
-// cost more per flop (each B fragment serves fewer MFMAs, each A fragment fewer
-// tiles).  The model: workgroups run in rounds of (CUs x workgroups per CU, from the
-// kernel's occupancy); a round costs (workgroups per CU) x (tile work) x (the shape's
-// relative cost per flop), a last round of at most one workgroup per CU 0.67 of that
-// where a CU holds two (a workgroup alone on its CU runs faster than two sharing it);
-// at one workgroup per CU a last round costs a full one (each workgroup already has
-// its CU alone).
-// The relative costs are fitted to shape-by-shape timings on MI355X (Q4_0 / Q8_0,
-// M = 128..2048, 1024..28672 rows): on bf16 x the model picks the fastest shape in
-// 66 of 70 cases (worst +12%); split x, whose steps run twice the MFMAs, has costs of
-// its own and picks the fastest in 39 of 40 (worst +0.6%).  Fixed per shape, so a
-// row's bits depend only on m and the weight.  A shape with per_cu < 0 is not built
-// for the instance: Q6_K on bf16 x has no 128 x 96 tiles (its super-block sums take
-// 96 more registers and would spill), and split x no 64 x 96 tiles (64 x 64 ran
-// faster or within 0.6% at every measured size).
-int choose_shape(const Weight& w, int64_t m, const int (&per_cu)[4], bool split_x) {
-    static const int bm[4] = {128, 128, 64, 64}, wt[4] = {3, 2, 3, 2};
-    static const double cost_per_flop[2][4] = {{1.00, 1.10, 1.25, 1.35},   // bf16 x
-                                               {1.00, 1.10, 1.40, 1.20}};  // split x
-    const int64_t cus = 256;
+// Launch shapes: eight waves each, as column slices x K parts.
+//   0: 128 x 192 tiles, 4 x 2 waves, 3 weight tiles per wave   3:  64 x 128, 4 x 2 waves, 2 tiles
+//   1: 128 x 128, 4 x 2 waves, 2 tiles                        4:  64 x  64, 2 x 4 waves, 2 tiles
+//   2:  64 x  96, 2 x 4 waves, 3 tiles                        5:  64 x  32, 1 x 8 waves, 2 tiles
+constexpr int kShapes = 6;
+constexpr int kShapeRows[kShapes] = {128, 128, 64, 64, 64, 64};
+constexpr int kShapeTiles[kShapes] = {12, 8, 6, 8, 4, 2};  // weight tiles (16 columns) per workgroup
+// Launch shape by problem size.  Few and large workgroups leave CUs idle or a last round
+// part-filled; small ones cost more per flop (each B fragment serves fewer MFMAs, each A
+// fragment fewer tiles).  The model: workgroups run in rounds of 256 CUs x one (or two,
+// where the kernel's registers let two share a CU: 64 x 128 and 64 x 64); a round costs
+// the shape's time per K element, measured on MI355X over 15 weight shapes x 100..1024
+// rows (Q4_0 / Q8_0 / Q4_K, and Q6_K, whose blocks run two to four MFMAs, on its own):
+// kOne for one workgroup on a CU, kTwo for two, plus kExtra for a workgroup's start and
+// K-part sums where that decides (64 x 96 at short K).  It picks the fastest shape or one
+// within 3% of it at every size measured; e.g. fp32 x, 100 rows of Q8_0 4096 x 11008: 64 x
+// 32 40.3 us, 64 x 64 63.1, 64 x 96 78.8, 64 x 128 97.7, 128 x 128 155, 128 x 192 216; bf16
+// x, 1024 rows of Q4_0 28672 x 8192: 128 x 192 566 us, 128 x 128 585, 64 x 128 622, 64 x 64
+// 696.  Fixed per shape, so a row's bits depend only on m and the weight.  A shape with
+// per_cu < 0 is not built for the instance: Q6_K on bf16 x has no 128 x 192 tiles (its
+// super-block sums would not fit the registers).
+int choose_shape(const Weight& w, int64_t m, const int (&per_cu)[kShapes], bool split_x) {
+    static const double kOne[4][kShapes] = {{13.8, 9.8, 4.8, 5.9, 3.4, 2.0},      // bf16 x
+                                            {0.0, 14.3, 8.2, 10.3, 5.7, 3.4},     // bf16 x, Q6_K
+                                            {21.8, 15.6, 7.0, 8.25, 5.2, 3.0},    // split x
+                                            {34.0, 23.2, 11.3, 14.4, 7.8, 4.9}};  // split x, Q6_K
+    static const double kTwo[2][kShapes] = {{0, 0, 0, 10.8, 5.9, 0}, {0, 0, 0, 15.9, 8.8, 0}};
+    static const double kExtra[4] = {500.0, 500.0, 1000.0, 1700.0};  // ns, shape 2
+    constexpr int64_t kCus = 256;
+    const int row = (split_x ? 2 : 0) + (w.type == OPENMINI_QMM_Q6_K ? 1 : 0);
     int best = -1;
     double best_cost = 0.0;
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < kShapes; ++i) {
         if (per_cu[i] < 0) continue;
-        const int spc = per_cu[i] > 0 ? per_cu[i] : 1;
-        const int64_t wgs = (w.n_tiles + 2 * wt[i] - 1) / (2 * wt[i]) * ((m + bm[i] - 1) / bm[i]);
-        const int64_t slots = cus * spc;
-        const double round = (double)spc * bm[i] * wt[i] * cost_per_flop[split_x][i] * (spc == 1 ? 1.2 : 1.0);
-        double cost = (double)(wgs / slots) * round;
-        if (wgs % slots) cost += round * (spc > 1 && wgs % slots <= cus ? 0.67 : 1.0);
+        const int64_t wgs = (w.n_tiles + kShapeTiles[i] - 1) / kShapeTiles[i] * ((m + kShapeRows[i] - 1) / kShapeRows[i]);
+        const double one = kOne[row][i];
+        const bool pairs = per_cu[i] >= 2 && kTwo[split_x][i] > 0.0;
+        const double full = pairs ? kTwo[split_x][i] : one;
+        const int64_t slots = pairs ? 2 * kCus : kCus, left = wgs % slots;
+        double cost = ((double)(wgs / slots) * full + (left > kCus ? full : left ? one : 0.0)) * (double)w.k;
+        if (i == 2) cost += kExtra[row];
         if (best < 0 || cost < best_cost) best = i, best_cost = cost;
     }
     return best;
@@ -629,57 +717,47 @@ int blocks_per_cu(const void* kernel, int threads) {
 template <int kFmt, bool kX2>
 constexpr bool kWideTiles = kFmt != OPENMINI_QMM_Q6_K || kX2;
 
-template <int kFmt, bool kGate, bool kX2>
-int shape0_per_cu() {
-    if constexpr (kWideTiles<kFmt, kX2>)
-        return blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 2, 2, 2, 3, kGate, kX2>, 256);
-    else
-        return -1;
-}
-
-// Shape 2 is built for bf16 x only.
-template <int kFmt, bool kGate, bool kX2>
-int shape2_per_cu() {
-    if constexpr (!kX2)
-        return blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 4, 2, 3, kGate, kX2>, 512);
-    else
-        return -1;
-}
-
-// Workgroups per CU of the four shapes' kernels (queried once per instantiation).
-template <int kFmt, bool kGate, bool kX2>
-const int (&shape_occupancy())[4] {
-    static const int per_cu[4] = {
-        shape0_per_cu<kFmt, kGate, kX2>(),
-        blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 2, 2, 2, 2, kGate, kX2>, 256),
-        shape2_per_cu<kFmt, kGate, kX2>(),
-        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 4, 2, 2, kGate, kX2>, 512)};
+// Workgroups per CU of the shapes' kernels (queried once per instantiation; -1: not built).
+template <int kFmt, bool kX2>
+const int (&shape_occupancy())[kShapes] {
+    auto wide = [] {
+        if constexpr (kWideTiles<kFmt, kX2>)
+            return blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 4, 2, 3, kX2>, 512);
+        else
+            return -1;
+    };
+    static const int per_cu[kShapes] = {wide(),
+                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 4, 2, 2, kX2>, 512),
+                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 4, 3, kX2>, 512),
+                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 4, 2, 2, kX2>, 512),
+                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 4, 2, kX2>, 512),
+                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 1, 8, 2, kX2>, 512)};
     return per_cu;
 }
 
-template <int kFmt, bool kGate, bool kX2>
-hipError_t launch_kind(const Weight& w, const uint16_t* x, const int* x_exp, float* y, int64_t m, int64_t kx,
+template <int kFmt, bool kX2>
+hipError_t launch_kind(const Weight& w, const uint16_t* x, const int* x_exp, float* y, int64_t m, bool gate,
                        hipStream_t s) {
-    switch (choose_shape(w, m, shape_occupancy<kFmt, kGate, kX2>(), kX2)) {
+    switch (choose_shape(w, m, shape_occupancy<kFmt, kX2>(), kX2)) {
     case 0:
-        if constexpr (kWideTiles<kFmt, kX2>) return launch_shape<kFmt, 128, 2, 2, 2, 3, kGate, kX2>(w, x, x_exp, y, m, kx, s);
+        if constexpr (kWideTiles<kFmt, kX2>) return launch_shape<kFmt, 128, 4, 2, 3, kX2>(w, x, x_exp, y, m, gate, s);
         return hipErrorInvalidValue;
-    case 1: return launch_shape<kFmt, 128, 2, 2, 2, 2, kGate, kX2>(w, x, x_exp, y, m, kx, s);
-    case 2:
-        if constexpr (!kX2) return launch_shape<kFmt, 64, 2, 4, 2, 3, kGate, kX2>(w, x, x_exp, y, m, kx, s);
-        return hipErrorInvalidValue;
-    default: return launch_shape<kFmt, 64, 2, 4, 2, 2, kGate, kX2>(w, x, x_exp, y, m, kx, s);
+    case 1: return launch_shape<kFmt, 128, 4, 2, 2, kX2>(w, x, x_exp, y, m, gate, s);
+    case 2: return launch_shape<kFmt, 64, 2, 4, 3, kX2>(w, x, x_exp, y, m, gate, s);
+    case 3: return launch_shape<kFmt, 64, 4, 2, 2, kX2>(w, x, x_exp, y, m, gate, s);
+    case 4: return launch_shape<kFmt, 64, 2, 4, 2, kX2>(w, x, x_exp, y, m, gate, s);
+    default: return launch_shape<kFmt, 64, 1, 8, 2, kX2>(w, x, x_exp, y, m, gate, s);
     }
 }
 
-template <bool kGate, bool kX2>
-hipError_t launch_type(const Weight& w, const uint16_t* x, const int* x_exp, float* y, int64_t m, int64_t kx,
+template <bool kX2>
+hipError_t launch_type(const Weight& w, const uint16_t* x, const int* x_exp, float* y, int64_t m, bool gate,
                        hipStream_t s) {
     switch (w.type) {
-    case OPENMINI_QMM_Q4_0: return launch_kind<OPENMINI_QMM_Q4_0, kGate, kX2>(w, x, x_exp, y, m, kx, s);
-    case OPENMINI_QMM_Q8_0: return launch_kind<OPENMINI_QMM_Q8_0, kGate, kX2>(w, x, x_exp, y, m, kx, s);
-    case OPENMINI_QMM_Q4_K: return launch_kind<OPENMINI_QMM_Q4_K, kGate, kX2>(w, x, x_exp, y, m, kx, s);
-    case OPENMINI_QMM_Q6_K: return launch_kind<OPENMINI_QMM_Q6_K, kGate, kX2>(w, x, x_exp, y, m, kx, s);
+    case OPENMINI_QMM_Q4_0: return launch_kind<OPENMINI_QMM_Q4_0, kX2>(w, x, x_exp, y, m, gate, s);
+    case OPENMINI_QMM_Q8_0: return launch_kind<OPENMINI_QMM_Q8_0, kX2>(w, x, x_exp, y, m, gate, s);
+    case OPENMINI_QMM_Q4_K: return launch_kind<OPENMINI_QMM_Q4_K, kX2>(w, x, x_exp, y, m, gate, s);
+    case OPENMINI_QMM_Q6_K: return launch_kind<OPENMINI_QMM_Q6_K, kX2>(w, x, x_exp, y, m, gate, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -690,49 +768,94 @@ hipError_t launch_type(const Weight& w, const uint16_t* x, const int* x_exp, flo
 // (exact in fp32, at most 13 bits, |lo| < 2^-10 |x'|) rounded to nearest fp16: the
 // pair carries x' to within 2^-22 |x'|, and to within 2^-25 absolute (2^-39 of the
 // row maximum) for elements more than 2^17 below it, where lo is an fp16 subnormal.
-// Written per 32-element block as 32 hi then 32 lo (x2 row = 2 k fp16), e in
-// x_exp[m].  A row holding inf or NaN is written as NaN (hi) and 0 (lo) with e = 0,
-// so every output of that row is NaN (the decode GEMVs do the same).  One workgroup
-// per row; x rows 16-byte aligned (k % 32 == 0).
-__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, uint16_t* __restrict__ x2,
-                                                         int* __restrict__ x_exp, int k) {
-    __shared__ uint32_t wave_max[4];
-    const size_t row = blockIdx.x;
-    const float4* xr = reinterpret_cast<const float4*>(x + row * (size_t)k);
-    const int quads = k / 4;
+// e goes to x_exp[m].  A row holding inf or NaN is written as NaN (hi) and 0 (lo) with
+// e = 0, so every output of that row is NaN (the decode GEMVs do the same).
+//
+// Written in the order the GEMM's fragments take it, so that its copies are contiguous:
+// per 16-row tile (the last one of r <= 16 rows) and 32-element block, r x 4 pieces of 8
+// hi values, piece kq * r + i = elements 8 kq .. 8 kq + 7 of row i, then the lo values
+// the same way.  With `nib` a piece holds its elements in the order (0, 2, 1, 3, 4, 6, 5,
+// 7), which makes the nibble codes three operations cheaper to build (codes_q4_perm).
+// One workgroup per row, which it reads once into registers (K <= 16384; the rest twice).
+// Rows go to workgroups so that a tile's 16 rows, which share cache lines of x2, run on
+// one XCD (workgroups are dealt out to the 8 XCDs in turn).  x rows 16-byte aligned
+// (k % 32 == 0).
+constexpr int kSplitThreads = 512;
+constexpr int kSplitHeld = 4;  // pieces of 8 elements a thread holds
+__global__ __launch_bounds__(kSplitThreads) void split_rows_kernel(const float* __restrict__ x,
+                                                                   uint16_t* __restrict__ x2,
+                                                                   int* __restrict__ x_exp, int m, int k, int nib) {
+    __shared__ uint32_t wave_max[kSplitThreads / 64];
+    const int tile = (int)(blockIdx.x >> 7) * 8 + (int)(blockIdx.x & 7), ri = (int)(blockIdx.x >> 3) & 15;
+    const int row = tile * 16 + ri;
+    if (row >= m) return;  // uniform
+    const float4* xr = reinterpret_cast<const float4*>(x + (size_t)row * k);
+    const int pieces = k / 8;
+    float4 h[kSplitHeld][2];
+    auto load = [&](int p, float4* v) {
+        v[0] = xr[2 * p];
+        v[1] = xr[2 * p + 1];
+    };
     uint32_t mx = 0;  // largest |x| as bits (inf / NaN above every finite value)
-    for (int i = (int)threadIdx.x; i < quads; i += 256) {
-        const float4 v = xr[i];
-        mx = max(max(mx, __float_as_uint(v.x) & 0x7FFFFFFFu), __float_as_uint(v.y) & 0x7FFFFFFFu);
-        mx = max(max(mx, __float_as_uint(v.z) & 0x7FFFFFFFu), __float_as_uint(v.w) & 0x7FFFFFFFu);
+    auto fold = [&](const float4* v) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            mx = max(max(mx, __float_as_uint(v[q].x) & 0x7FFFFFFFu), __float_as_uint(v[q].y) & 0x7FFFFFFFu);
+            mx = max(max(mx, __float_as_uint(v[q].z) & 0x7FFFFFFFu), __float_as_uint(v[q].w) & 0x7FFFFFFFu);
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < kSplitHeld; ++c) {
+        const int p = (int)threadIdx.x + c * kSplitThreads;
+        h[c][0] = h[c][1] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (p < pieces) load(p, h[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < kSplitHeld; ++c) fold(h[c]);
+    for (int p = (int)threadIdx.x + kSplitHeld * kSplitThreads; p < pieces; p += kSplitThreads) {
+        float4 v[2];
+        load(p, v);
+        fold(v);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
     if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = mx;
     __syncthreads();
-    mx = max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
+#pragma unroll
+    for (int w = 0; w < kSplitThreads / 64; ++w) mx = max(mx, wave_max[w]);
     const bool bad = mx >= 0x7F800000u;
     // max |x| in [2^(f - 1), 2^f): e = 15 - f puts it in [2^14, 2^15)
     const int e = (bad || mx == 0) ? 0 : 15 - __builtin_amdgcn_frexp_expf(__uint_as_float(mx));
-    uint16_t* out = x2 + row * (size_t)(2 * k);
-    for (int i = (int)threadIdx.x; i < quads; i += 256) {
-        const float4 v = xr[i];
-        uint2 hi, lo;
-        if (bad) {
-            hi = make_uint2(0x7E007E00u, 0x7E007E00u);  // fp16 NaN
-            lo = make_uint2(0u, 0u);
-        } else {
-            const float a0 = __builtin_amdgcn_ldexpf(v.x, e), a1 = __builtin_amdgcn_ldexpf(v.y, e);
-            const float a2 = __builtin_amdgcn_ldexpf(v.z, e), a3 = __builtin_amdgcn_ldexpf(v.w, e);
-            const auto h01 = __builtin_amdgcn_cvt_pkrtz(a0, a1), h23 = __builtin_amdgcn_cvt_pkrtz(a2, a3);
-            hi = make_uint2(__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23));
-            const f16x2 l01 = {(_Float16)(a0 - (float)h01[0]), (_Float16)(a1 - (float)h01[1])};
-            const f16x2 l23 = {(_Float16)(a2 - (float)h23[0]), (_Float16)(a3 - (float)h23[1])};
-            lo = make_uint2(__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23));
+    const int rows = min(16, m - tile * 16);
+    uint4* out = reinterpret_cast<uint4*>(x2 + (size_t)tile * 32 * k);  // 16-byte pieces
+    auto put = [&](int p, const float4* q) {
+        float v[8] = {q[0].x, q[0].y, q[0].z, q[0].w, q[1].x, q[1].y, q[1].z, q[1].w};
+        if (nib) {
+            v[1] = q[0].z; v[2] = q[0].y;
+            v[5] = q[1].z; v[6] = q[1].y;
         }
-        const int b = i >> 3, e0 = (i & 7) * 4;  // 32-element block, element within it
-        *reinterpret_cast<uint2*>(out + b * 64 + e0) = hi;
-        *reinterpret_cast<uint2*>(out + b * 64 + 32 + e0) = lo;
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float a = __builtin_amdgcn_ldexpf(v[2 * i], e), b = __builtin_amdgcn_ldexpf(v[2 * i + 1], e);
+            const auto t = __builtin_amdgcn_cvt_pkrtz(a, b);
+            const f16x2 l = {(_Float16)(a - (float)t[0]), (_Float16)(b - (float)t[1])};
+            hi[i] = bad ? 0x7E007E00u : __builtin_bit_cast(uint32_t, t);  // fp16 NaN
+            lo[i] = bad ? 0u : __builtin_bit_cast(uint32_t, l);
+        }
+        uint4* at = out + (size_t)(p >> 2) * 8 * rows + (p & 3) * rows + ri;
+        at[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        at[4 * rows] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    };
+#pragma unroll
+    for (int c = 0; c < kSplitHeld; ++c) {
+        const int p = (int)threadIdx.x + c * kSplitThreads;
+        if (p < pieces) put(p, h[c]);
+    }
+    for (int p = (int)threadIdx.x + kSplitHeld * kSplitThreads; p < pieces; p += kSplitThreads) {
+        float4 v[2];
+        load(p, v);
+        put(p, v);
     }
     if (threadIdx.x == 0) x_exp[row] = e;
 }
@@ -804,10 +927,10 @@ __global__ __launch_bounds__(512) void gemm_ceiling_kernel(int blocks, float* __
 
 template <int kFmt>
 hipError_t launch_ceiling(int64_t m, int64_t n_tiles, int64_t k, float* sink, hipStream_t s) {
-    // the grid, workgroup and K split of launch_kind's two shapes
+    // the grid, workgroup and K split of the launch shapes 128 x 192 and (few rows) 64 x 96
     const bool small = m <= kBMMax;
-    const int bm = small ? 64 : 128, threads = small ? 512 : 256, parts = small ? 4 : 2;
-    const int64_t bt = 2 * kCeilWT;  // weight tiles per workgroup (2 column slices)
+    const int bm = small ? 64 : 128, threads = 512, parts = small ? 4 : 2;
+    const int64_t bt = (small ? 2 : 4) * kCeilWT;  // weight tiles per workgroup (column slices)
     const dim3 grid((unsigned)((n_tiles + bt - 1) / bt), (unsigned)((m + bm - 1) / bm));
     const int blocks = (int)((k / kQK + parts - 1) / parts);
     if (small)
@@ -827,36 +950,39 @@ hipError_t launch_gemm_ceiling(int type, int64_t m, int64_t n, int64_t k, float*
     return hipErrorInvalidValue;
 }
 
+// Rows of one launch: x offsets are 32-bit, so x stays below 2 GiB (row_bytes per row), and
+// the grid's y dimension counts at most 65535 tiles of 64 rows.
+static int64_t rows_of_launch(int64_t row_bytes) {
+    const int64_t rows = (((int64_t)1 << 31) - 1) / row_bytes, grid = (int64_t)65535 * 64;
+    return (rows < grid ? rows : grid) / kBMMax * kBMMax;
+}
+
 hipError_t launch_gemm_bf16(const Weight& w, const uint16_t* x, float* y, int64_t m, hipStream_t s,
                             bool gate_in_y) {
-    // x offsets are 32-bit: launches cover row ranges whose x is below 2 GiB.
-    const int64_t rows_per_launch = ((((int64_t)1 << 31) - 1) / (w.k * 2)) / kBMMax * kBMMax;
+    const int64_t rows_per_launch = rows_of_launch(w.k * 2);
     if (rows_per_launch <= 0) return hipErrorInvalidValue;  // one row tile of x exceeds 2 GiB
     for (int64_t m_off = 0; m_off < m; m_off += rows_per_launch) {
         const int64_t mm = m - m_off < rows_per_launch ? m - m_off : rows_per_launch;
         const uint16_t* xs = x + m_off * w.k;
         float* ys = y + m_off * w.n;
-        const hipError_t e = gate_in_y ? launch_type<true, false>(w, xs, nullptr, ys, mm, w.k, s)
-                                       : launch_type<false, false>(w, xs, nullptr, ys, mm, w.k, s);
+        const hipError_t e = launch_type<false>(w, xs, nullptr, ys, mm, gate_in_y, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
 int gemm_shape(const Weight& w, int64_t m, bool split_x) {
+    auto pick = [&](auto fmt) {
+        constexpr int kFmt = decltype(fmt)::value;
+        const int i = split_x ? choose_shape(w, m, shape_occupancy<kFmt, true>(), true)
+                              : choose_shape(w, m, shape_occupancy<kFmt, false>(), false);
+        return i > 3 ? 3 : i;  // by rows per workgroup and weight tiles per wave
+    };
     switch (w.type) {
-    case OPENMINI_QMM_Q4_0:
-        return split_x ? choose_shape(w, m, shape_occupancy<OPENMINI_QMM_Q4_0, false, true>(), split_x)
-                       : choose_shape(w, m, shape_occupancy<OPENMINI_QMM_Q4_0, false, false>(), split_x);
-    case OPENMINI_QMM_Q8_0:
-        return split_x ? choose_shape(w, m, shape_occupancy<OPENMINI_QMM_Q8_0, false, true>(), split_x)
-                       : choose_shape(w, m, shape_occupancy<OPENMINI_QMM_Q8_0, false, false>(), split_x);
-    case OPENMINI_QMM_Q4_K:
-        return split_x ? choose_shape(w, m, shape_occupancy<OPENMINI_QMM_Q4_K, false, true>(), split_x)
-                       : choose_shape(w, m, shape_occupancy<OPENMINI_QMM_Q4_K, false, false>(), split_x);
-    case OPENMINI_QMM_Q6_K:
-        return split_x ? choose_shape(w, m, shape_occupancy<OPENMINI_QMM_Q6_K, false, true>(), split_x)
-                       : choose_shape(w, m, shape_occupancy<OPENMINI_QMM_Q6_K, false, false>(), split_x);
+    case OPENMINI_QMM_Q4_0: return pick(std::integral_constant<int, OPENMINI_QMM_Q4_0>{});
+    case OPENMINI_QMM_Q8_0: return pick(std::integral_constant<int, OPENMINI_QMM_Q8_0>{});
+    case OPENMINI_QMM_Q4_K: return pick(std::integral_constant<int, OPENMINI_QMM_Q4_K>{});
+    case OPENMINI_QMM_Q6_K: return pick(std::integral_constant<int, OPENMINI_QMM_Q6_K>{});
     default: return -1;
     }
 }
@@ -865,11 +991,15 @@ size_t gemm_f32_workspace_bytes(int64_t m, int64_t k) {
     return (((size_t)m * (size_t)k * 4 + 255) & ~(size_t)255) + (size_t)m * 4;
 }
 
-hipError_t split_rows(const float* x, int64_t m, int64_t k, void* work, hipStream_t s) {
+hipError_t split_rows(const Weight& w, const float* x, int64_t m, void* work, hipStream_t s) {
+    const int64_t k = w.k;
     if (m <= 0 || m > INT32_MAX || k <= 0 || k % kQK != 0 || k > INT32_MAX / 2) return hipErrorInvalidValue;
     uint16_t* x2 = static_cast<uint16_t*>(work);
     int* x_exp = reinterpret_cast<int*>(static_cast<uint8_t*>(work) + (gemm_f32_workspace_bytes(m, k) - (size_t)m * 4));
-    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)m), dim3(256), 0, s, x, x2, x_exp, (int)k);
+    const int nib = w.type == OPENMINI_QMM_Q4_0 || w.type == OPENMINI_QMM_Q4_K;
+    const int64_t tiles = (m + 15) / 16;
+    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)((tiles + 7) / 8 * 128)), dim3(kSplitThreads), 0, s, x, x2, x_exp,
+                       (int)m, (int)k, nib);
     return hipGetLastError();
 }
 
@@ -878,15 +1008,14 @@ hipError_t launch_gemm_split(const Weight& w, const void* work, int64_t m, float
     const int* x_exp =
         reinterpret_cast<const int*>(static_cast<const uint8_t*>(work) + (gemm_f32_workspace_bytes(m, w.k) - (size_t)m * 4));
     const int64_t kx = 2 * w.k;  // fp16 elements per split row
-    const int64_t rows_per_launch = ((((int64_t)1 << 31) - 1) / (kx * 2)) / kBMMax * kBMMax;
+    const int64_t rows_per_launch = rows_of_launch(kx * 2);
     if (rows_per_launch <= 0) return hipErrorInvalidValue;
     for (int64_t m_off = 0; m_off < m; m_off += rows_per_launch) {
         const int64_t mm = m - m_off < rows_per_launch ? m - m_off : rows_per_launch;
         const uint16_t* xs = x2 + m_off * kx;
         const int* es = x_exp + m_off;
         float* ys = y + m_off * w.n;
-        const hipError_t e = gate_in_y ? launch_type<true, true>(w, xs, es, ys, mm, kx, s)
-                                       : launch_type<false, true>(w, xs, es, ys, mm, kx, s);
+        const hipError_t e = launch_type<true>(w, xs, es, ys, mm, gate_in_y, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

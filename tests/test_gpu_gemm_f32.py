@@ -269,3 +269,32 @@ def test_gemm_every_launch_shape(qmm, orc, qtype, split_x):
         seen.setdefault(shape, (N, M))
     expect = [0, 1, 3] if split_x else [1, 2, 3] if qtype == 14 else [0, 1, 2, 3]
     assert sorted(seen) == expect, seen
+
+
+@pytest.mark.parametrize("qtype,N,K,M", [
+    (Q4_0, 33, 32, 1), (Q8_0, 31, 96, 17),         # fewer K groups than K parts, a ragged last group
+    (Q4_0, 200, 1120, 63), (Q8_0, 65, 1120, 129),  # a part without a last group; a row past a tile
+    (Q4_K, 97, 768, 65), (Q6_K, 130, 768, 100),    # super-blocks across parts
+    (Q4_0, 4090, 96, 200), (Q8_0, 4100, 160, 130), (Q6_K, 4100, 256, 200),
+    (Q8_0, 8200, 96, 1000), (Q4_K, 11000, 256, 500), (Q6_K, 11000, 256, 400)])
+def test_gemm_tile_edges(qmm, orc, qtype, N, K, M):
+    """Every launch shape at the edges of its tiles, on bf16 and fp32 activations: rows and
+    columns past whole tiles, K parts of zero, one and unequal group counts.  The products
+    are exact, so the outputs differ from fp64 by fp32 sums of at most K / 32 block sums
+    of 32 terms: 1e-5 of the largest output is above 20 times that rounding."""
+    blocks = blocks_for(qtype, N, K, seed=0xFA0 + N + K + M)
+    x = synth.normal(0xFA1 + M, (M, K), 1.0)
+    w = qmm.QuantizedWeight(qtype, blocks, N, K)
+    rows = np.unique(np.concatenate([[0, M - 1], np.random.default_rng(N).integers(0, M, 6)]))
+    y = run_gemm_f32(qmm, w, x)
+    assert np.all(np.isfinite(y)), "unwritten (NaN) outputs"
+    ref = orc.linear_f64(qtype, blocks, N, K, x[rows])
+    assert np.max(np.abs(y[rows] - ref)) <= 1e-5 * np.max(np.abs(ref))
+    xb = synth.to_bf16_bits(x)
+    dx, dy = qmm.DeviceBuffer.from_numpy(xb), qmm.DeviceBuffer(M * N * 4)
+    dy.fill(0xFF)
+    w.gemm_bf16(dx, dy, M)
+    yb = dy.download(np.float32, (M, N))
+    assert np.all(np.isfinite(yb)), "unwritten (NaN) outputs"
+    refb = orc.linear_bf16x_f64(qtype, blocks, N, K, xb[rows])
+    assert np.max(np.abs(yb[rows] - refb)) <= 1e-5 * np.max(np.abs(refb))
