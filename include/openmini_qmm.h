@@ -183,8 +183,9 @@ int openmini_qmm_weight_info(const openmini_qweight_t* weight,
 
 /* Decode GEMV: y[batch, N] = x[batch, K] . W^T, fp32 activations, fp32 output.
  * Any batch >= 1.  Up to 3 rows: the single-row-tuned kernel; 4 or more: the
- * batched kernel, one pass over W per 16 rows, in which a row's result does not
- * depend on the other rows of the call nor on the batch size (bitwise).  Every
+ * batched kernels, one pass over W per 16 rows (17 to 64 rows: one pass for all on
+ * weights of at most 12288 rows), in which a row's result does not depend on the
+ * other rows of the call nor on the batch size (bitwise).  Every
  * weight type.
  * A weight of at most 8192 rows and K >= 4000 splits K of a batched call over two or
  * four workgroups per row tile; their partial sums and arrival counters live in a

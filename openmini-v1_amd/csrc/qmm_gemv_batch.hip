@@ -72,14 +72,14 @@ __device__ __forceinline__ float minus_half(uint32_t h, float x) {
     return r;
 }
 
-// 8 scaled activations -> fp16 hi and lo parts: hi = x' rounded toward zero to fp16
-// (11 significant bits for x' >= 2^-14), lo = x' - hi, exact in fp32, rounded toward
-// zero to fp16.
-__device__ __forceinline__ void split8(const float* v, int s, f16x8& hi, f16x8& lo) {
+// 8 activations scaled by f = 2^s -> fp16 hi and lo parts: hi = x' = x f rounded toward
+// zero to fp16 (11 significant bits for x' >= 2^-14), lo = x' - hi, exact in fp32, rounded
+// toward zero to fp16.  (A multiplication issues in half the cycles v_ldexp takes.)
+__device__ __forceinline__ void split8(const float* v, float f, f16x8& hi, f16x8& lo) {
     uint32_t h[4], l[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float a = __builtin_amdgcn_ldexpf(v[2 * j], s), b = __builtin_amdgcn_ldexpf(v[2 * j + 1], s);
+        const float a = v[2 * j] * f, b = v[2 * j + 1] * f;
         h[j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
         l[j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(minus_half<0>(h[j], a), minus_half<1>(h[j], b)));
     }
@@ -306,8 +306,10 @@ __global__ __launch_bounds__(64 * W) void gemv_batch_kernel(const uint8_t* __res
         m = quarter_max(m);
         if constexpr (kRep >= 2) m = fmaxf(m, row_ror<8>(m));  // the parts of a row: lanes li, li ^ 8
         if constexpr (kRep == 4) m = fmaxf(m, row_ror<4>(m));  // and li + 4, li + 12
-        // 2^e <= m < 2^(e+1), e = biased exponent - 127; s = 14 - e
-        const int sh = 141 - (int)(__float_as_uint(m) >> 23);
+        // 2^e <= m < 2^(e+1), e = biased exponent - 127; s = 14 - e, at most 126 so that 2^s is
+        // a number (a group that small keeps every bit: fp16's quantum 2^-24 is 2^-150 there)
+        const int sh = min(141 - (int)(__float_as_uint(m) >> 23), 126);
+        const float up = __builtin_amdgcn_ldexpf(1.0f, sh);
         if (kq == 0) my_scale[li] = __builtin_amdgcn_ldexpf(1.0f, -sh);
         if constexpr (F::kMin) {
             // the sums of the lane's activation blocks (the lane's 8 elements, then the
@@ -323,7 +325,7 @@ __global__ __launch_bounds__(64 * W) void gemv_batch_kernel(const uint8_t* __res
         }
         f16x8 ah[4], al[4];  // A operands of blocks 0..3 for the batch rows' lanes
 #pragma unroll
-        for (int tt = 0; tt < kXB; ++tt) split8(st.x[tt], sh, ah[tt], al[tt]);
+        for (int tt = 0; tt < kXB; ++tt) split8(st.x[tt], up, ah[tt], al[tt]);
 #pragma unroll
         for (int t = kXB; t < 4; ++t) {  // part t / kXB: lanes li + kPartRows * (t / kXB)
             if (t / kXB == 1) {
@@ -545,6 +547,384 @@ __global__ __launch_bounds__(64 * W) void gemv_batch_kernel(const uint8_t* __res
     }
 }
 
+// A K group's weights of kNT (weight, tile) pairs as loaded: chunk slot `lane` whole.
+template <int kFmt, int kNT>
+struct RawGroup {
+    using F = BFmt<kFmt>;
+    uint4 c[kNT][F::kQ8 ? 2 : 1];
+    uint2 hb[F::kQ6K ? kNT : 1];
+    uint32_t sc[kNT], dk[F::kKQ ? kNT : 1], mn[F::kMin ? kNT : 1], dm[F::kQ5 ? kNT : 1];
+};
+
+// The same as MFMA operands: codes (Q6_K: q * scale as hi, lo), block factors, block-minimum
+// offsets; the forms and reasons are gemv_batch_kernel's.
+template <int kFmt, int kNT>
+struct GroupOps {
+    using F = BFmt<kFmt>;
+    static constexpr bool kQ6 = F::kQ6K && !F::kQ5;
+    f16x8 b[kNT][4][kQ6 ? 2 : 1];
+    float f[kNT][kQ6 ? 1 : 4];
+    float os[F::kMin ? kNT : 1][4];
+};
+
+// ---- more than 16 rows in one pass over W ------------------------------------------
+//
+// kMG row groups of 16 activation rows (2 for up to 32 rows, else 4, those without rows
+// skipped) share a workgroup's weights: a K group's chunks
+// are loaded, transposed and converted once, then each row group's activations are
+// split and multiplied in turn, with the arithmetic and the order of gemv_batch_kernel (a
+// row's result is bitwise the same whichever kernel and row group it falls in: the waves
+// and K slices are the ones a 16-row call on the weight has, see choose_rows_shape).
+// The activations come through LDS: an item (K group, row group) is 16 rows x 512 bytes,
+// copied by buffer loads with an LDS destination -- whole 512-byte row spans, where
+// lanes that each load 32 bytes of their own row touch 16 lines per load -- two items
+// ahead and without registers.  LDS position p of a row holds its 16-byte segment p ^
+// (row % 8), so the reads of a lane's 8 elements are bank-conflict free.  Rows past the
+// batch and elements past K read zero (out-of-range buffer offsets).
+// What bounds it: VALU issue (the split, about 150 operations per item, and 20 per tile
+// and item).  Q4_K 11008 x 4096, 40 rows: 34.8 us in three
+// 16-row passes -> 22.6; 64 rows 49.7 -> 27.1; Q8_0 41.6 -> 27.5, 56.7 -> 32.0; Q4_0 4096 x
+// 4096, 64 rows 34.8 -> 17.8.
+template <int kFmt, int T, int W, int kNW, int kRH, int kMG>
+__global__ __launch_bounds__(64 * W * kRH, 2) void gemv_rows_kernel(const uint8_t* __restrict__ w0,
+                                                              const uint8_t* __restrict__ w1,
+                                                              const float* __restrict__ x, float* __restrict__ y,
+                                                              int n_rows, int n_tiles, int groups, int k, int batch) {
+    static_assert(kMG == 1 || kMG % 2 == 0, "the items of a K group start in slot 0, or alternate");
+    constexpr int kNT = kNW * T;
+    using F = BFmt<kFmt>;
+    constexpr int kCB = F::kCB;
+    constexpr int kCodeBytes = kTileEntries * kCB;
+    constexpr int kChunk = F::kChunk;
+    constexpr bool kQ6 = F::kQ6K && !F::kQ5;
+    constexpr int kCopies = 8;           // 1 KB copies per item
+    constexpr int kItemB = kCopies * 1024;
+    // One array per slot: the compiler then sees that a copy into one does not alias the
+    // reads of the other.
+    __shared__ __attribute__((aligned(16))) uint8_t slot0[W * kRH * kItemB];
+    __shared__ __attribute__((aligned(16))) uint8_t slot1[W * kRH * kItemB];
+    // per wave: 16 range scales, then (block minimum) 4 blocks x 16 activation-block sums
+    __shared__ __attribute__((aligned(16))) float scr[W * kRH][16 + (F::kMin ? 64 : 0)];
+    static_assert(kNT * 1024 <= kItemB, "a wave's partial sums of one row group fit its slot");
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, kq = lane >> 4;
+    const int tile0 = (int)blockIdx.x * T;
+    const int kw = wave % W, rh = wave / W;  // K slice, row half
+    const int row0 = rh * kMG * 16;          // this wave's first row
+    const float* __restrict__ xw = x + (size_t)row0 * k;
+    const int wrows = batch - row0;
+    // eight waves: two halves of four, as gemv_batch_kernel cuts K
+    constexpr int kWH = W == 8 ? 4 : W;
+    const int hs0 = (int)((int64_t)groups * (kw / kWH) / (W / kWH));
+    const int hsn = (int)((int64_t)groups * (kw / kWH + 1) / (W / kWH)) - hs0;
+    const int g0 = hs0 + (int)((int64_t)hsn * (kw % kWH) / kWH);
+    const int g1 = hs0 + (int)((int64_t)hsn * (kw % kWH + 1) / kWH);
+
+    const __amdgpu_buffer_rsrc_t w_rs0 = make_rsrc(w0, (uint32_t)n_tiles * groups * kChunk);
+    const __amdgpu_buffer_rsrc_t w_rs1 = make_rsrc(kNW == 2 ? w1 : w0, (uint32_t)n_tiles * groups * kChunk);
+    uint32_t tile_off[T];
+#pragma unroll
+    for (int i = 0; i < T; ++i) tile_off[i] = (uint32_t)min(tile0 + i, n_tiles - 1) * groups * kChunk;
+    float* my_scale = scr[wave];
+    float* my_sums = scr[wave] + 16;
+
+    // Copy j of an item: rows 2 j, 2 j + 1; this lane's 16-byte segment and row in it.
+    uint32_t x_lane[kCopies], x_elem[4];
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j) {
+        const uint32_t r = 2 * j + (lane >> 5), seg = (uint32_t)(lane & 31) ^ (r & 7);
+        x_lane[j] = (r * (uint32_t)k + seg * 4) * 4u;
+        x_elem[j & 3] = seg * 4;  // rows 8 apart share the segment order
+    }
+    const int read0 = li * 512 + ((kq * 2) ^ (li & 7)) * 16;  // in an item: this lane's segment 2 kq
+    auto copy_item = [&](int gv, int mg, uint8_t* slot) {
+        const int g = __builtin_amdgcn_readfirstlane(gv);  // uniform: in an SGPR, or each copy gets a loop
+        uint32_t left = (uint32_t)(k - g * 128);
+        asm volatile("" : "+s"(left));  // offsets of its own for each copy: shared ones would hold registers
+        // a resource per row group: rows past the batch are out of its range
+        const int rows = __builtin_amdgcn_readfirstlane(min(max(wrows - mg * 16, 0), 16));
+        const __amdgpu_buffer_rsrc_t x_rs = make_rsrc(xw + (size_t)mg * 16 * k, (uint32_t)rows * (uint32_t)k * 4u);
+        // Segments past K get an out-of-range offset: bit 31 where left - 1 - element is negative.
+        // The group's offset stays inside the row (it is not range-checked).
+        uint32_t past[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) past[j] = (left - 1u - x_elem[j]) & 0x80000000u;
+#pragma unroll
+        for (int j = 0; j < kCopies; ++j)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                x_rs, (__attribute__((address_space(3))) void*)(slot + wave * kItemB + j * 1024), 16,
+                x_lane[j] | past[j & 3], (uint32_t)g * 512u, 0, 0);
+    };
+
+    using Raw = RawGroup<kFmt, kNT>;
+    using Ops = GroupOps<kFmt, kNT>;
+    constexpr int kRawLoads =
+        kNT * (1 + (F::kQ8 ? 1 : 0) + (F::kQ6K ? 1 : 0) + 1 + (F::kKQ ? 1 : 0) + (F::kQ41 ? 1 : 0) + (F::kQ5 ? 2 : 0));
+    static_assert(2 * kRawLoads + kCopies <= 63, "vmcnt counts up to 63");
+    auto load_raw = [&](Raw& R, int g) {
+#pragma unroll
+        for (int i = 0; i < kNT; ++i) {
+            const __amdgpu_buffer_rsrc_t rs = i / T == 0 ? w_rs0 : w_rs1;
+            const uint32_t soff = tile_off[i % T] + (uint32_t)g * kChunk;
+            R.c[i][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * kCB, soff, 0));
+            if constexpr (F::kQ8)
+                R.c[i][1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * kCB + 16, soff, 0));
+            if constexpr (F::kQ5)
+                R.hb[i].x = __builtin_amdgcn_raw_buffer_load_b8(rs, kQ5KQhOff + lane, soff, 0);
+            else if constexpr (F::kQ6K)
+                R.hb[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, kCodeBytes + lane * 8, soff, 0));
+            if constexpr (F::kQ4K || F::kQ5)
+                R.sc[i] = __builtin_amdgcn_raw_buffer_load_b8(rs, F::kScaleOff + lane, soff, 0);
+            else
+                R.sc[i] = __builtin_amdgcn_raw_buffer_load_b16(rs, F::kScaleOff + lane * 2, soff, 0);
+            if constexpr (F::kKQ) R.dk[i] = __builtin_amdgcn_raw_buffer_load_b16(rs, F::kDOff + li * 2, soff, 0);
+            if constexpr (F::kQ41) R.mn[i] = __builtin_amdgcn_raw_buffer_load_b16(rs, kQ41MinOff + lane * 2, soff, 0);
+            if constexpr (F::kQ5) {
+                R.mn[i] = __builtin_amdgcn_raw_buffer_load_b8(rs, kQ5KMinOff + lane, soff, 0);
+                R.dm[i] = __builtin_amdgcn_raw_buffer_load_b16(rs, kQ5KDminOff + li * 2, soff, 0);
+            }
+        }
+    };
+
+    auto convert = [&](Ops& O, const Raw& R) {
+#pragma unroll
+        for (int i = 0; i < kNT; ++i) {
+            uint32_t e[4], o[4];
+            if constexpr (!F::kQ8) {
+                e[0] = R.c[i][0].x; e[1] = R.c[i][0].y; e[2] = R.c[i][0].z; e[3] = R.c[i][0].w;
+                transpose4(e[0], e[1], e[2], e[3]);
+                if constexpr (F::kQ5) {
+                    float hb4[4];
+                    broadcast4(__uint_as_float(R.hb[i].x), hb4);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) o[t] = __float_as_uint(hb4[t]);
+                } else if constexpr (F::kQ6K) {
+                    o[0] = R.hb[i].x; o[1] = R.hb[i].x; o[2] = R.hb[i].y; o[3] = R.hb[i].y;
+                    transpose4(o[0], o[1], o[2], o[3]);
+                }
+            } else {
+                e[0] = R.c[i][0].x; o[0] = R.c[i][0].y; e[1] = R.c[i][0].z; o[1] = R.c[i][0].w;
+                e[2] = R.c[i][1].x; o[2] = R.c[i][1].y; e[3] = R.c[i][1].z; o[3] = R.c[i][1].w;
+                transpose4(e[0], e[1], e[2], e[3]);
+                transpose4(o[0], o[1], o[2], o[3]);
+            }
+            if constexpr (kQ6) {
+                float sw[4];
+                broadcast4(__uint_as_float(R.sc[i]), sw);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const f16x8 b = codes_q6(e[t], o[t], kq);
+                    const _Float16 sc = (_Float16)(float)(int8_t)((__float_as_uint(sw[t]) >> ((kq >> 1) * 8)) & 0xFFu);
+                    const f16x8 s8 = f16x8{sc, sc, sc, sc, sc, sc, sc, sc};
+                    O.b[i][t][0] = b * s8;
+                    O.b[i][t][1] = __builtin_elementwise_fma(b, s8, -O.b[i][t][0]);
+                }
+                O.f[i][0] = f16_bits_to_f32((uint16_t)R.dk[i]);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    if constexpr (F::kNib)
+                        O.b[i][t][0] = codes_q4_perm(e[t]);  // the activations are read in its order
+                    else if constexpr (F::kQ5)
+                        O.b[i][t][0] = codes_q5(e[t], o[t]);
+                    else
+                        O.b[i][t][0] = codes_q8(e[t], o[t]);
+                }
+                if constexpr (F::kQ4K)
+                    broadcast4(f16_bits_to_f32((uint16_t)R.dk[i]) * (float)(R.sc[i] & 0xFFu), O.f[i]);
+                else if constexpr (F::kQ5)
+                    broadcast4(f16_bits_to_f32((uint16_t)R.dk[i]) * (float)(int8_t)(R.sc[i] & 0xFFu), O.f[i]);
+                else
+                    broadcast4(f16_bits_to_f32((uint16_t)R.sc[i]), O.f[i]);
+                if constexpr (F::kQ41)
+                    broadcast4(fmaf(8.0f, f16_bits_to_f32((uint16_t)R.sc[i]), f16_bits_to_f32((uint16_t)R.mn[i])), O.os[i]);
+                if constexpr (F::kQ5) broadcast4(f16_bits_to_f32((uint16_t)R.dm[i]) * (float)R.mn[i], O.os[i]);
+            }
+        }
+    };
+
+    f32x4 acc[kMG][kNT];
+#pragma unroll
+    for (int m = 0; m < kMG; ++m)
+#pragma unroll
+        for (int i = 0; i < kNT; ++i) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // One item: read, split and multiply (gemv_batch_kernel's compute).
+    auto fence = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto item = [&](const Ops& O, int mg, uint8_t* slot, int ahead, int next_g, int next_mg) {
+        fence();
+        // this item's copies have landed: at most the loads issued after them -- the next
+        // item's copies and `ahead` groups' weights -- are out
+        if (ahead == 0)
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(kCopies));
+        else if (ahead == 1)
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(kCopies + kRawLoads));
+        else
+            __builtin_amdgcn_s_waitcnt(vmcnt_only(kCopies + 2 * kRawLoads));
+        fence();
+        float v[4][8];
+        const uint8_t* at0 = slot + wave * kItemB + read0;
+        const uint8_t* at1 = slot + wave * kItemB + (read0 ^ 16);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {  // segments 8 t + 2 kq, 8 t + 2 kq + 1
+            const float4 a = *reinterpret_cast<const float4*>(at0 + t * 128);
+            const float4 b = *reinterpret_cast<const float4*>(at1 + t * 128);
+            if constexpr (F::kNib) {  // codes_q4_perm's element order
+                v[t][0] = a.x; v[t][1] = a.z; v[t][2] = a.y; v[t][3] = a.w;
+                v[t][4] = b.x; v[t][5] = b.z; v[t][6] = b.y; v[t][7] = b.w;
+            } else {
+                v[t][0] = a.x; v[t][1] = a.y; v[t][2] = a.z; v[t][3] = a.w;
+                v[t][4] = b.x; v[t][5] = b.y; v[t][6] = b.z; v[t][7] = b.w;
+            }
+        }
+        fence();
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slot may be overwritten
+        fence();
+        copy_item(next_g, next_mg, slot);
+        fence();
+        if (mg * 16 >= wrows) return;  // uniform: no rows in this group
+        float m = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(v[t][j]));
+        m = quarter_max(m);
+        const int sh = min(141 - (int)(__float_as_uint(m) >> 23), 126);
+        const float up = __builtin_amdgcn_ldexpf(1.0f, sh);
+        if (kq == 0) my_scale[li] = __builtin_amdgcn_ldexpf(1.0f, -sh);
+        if constexpr (F::kMin) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                float s = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) s += v[t][j];
+                s = quarter_sum(s);
+                if (kq == 0) my_sums[t * 16 + li] = s;
+            }
+        }
+        f16x8 ah[4], al[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) split8(v[t], up, ah[t], al[t]);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const f32x4 rs = *reinterpret_cast<const f32x4*>(my_scale + kq * 4);
+        f32x4 bs[4];
+        if constexpr (F::kMin) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) bs[t] = *reinterpret_cast<const f32x4*>(my_sums + t * 16 + kq * 4);
+        }
+#pragma unroll
+        for (int i = 0; i < kNT; ++i) {
+            if constexpr (kQ6) {
+                f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], O.b[i][t][0], d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t], O.b[i][t][0], d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], O.b[i][t][1], d, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t], O.b[i][t][1], d, 0, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[mg][i][r] = fmaf(d[r], rs[r] * O.f[i][0], acc[mg][i][r]);
+            } else {
+                f32x4 gs = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[t], O.b[i][t][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[t], O.b[i][t][0], d, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) gs[r] = fmaf(d[r], O.f[i][t], gs[r]);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[mg][i][r] = fmaf(gs[r], rs[r], acc[mg][i][r]);
+                if constexpr (F::kMin) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[mg][i][r] = fmaf(O.os[i][t], bs[t][r], acc[mg][i][r]);
+                }
+            }
+        }
+        // the next item rewrites my_scale after these reads (in-order LDS per wave)
+    };
+
+    if (g0 < g1 && wrows > 0) {  // uniform per wave
+        Raw raw;
+        load_raw(raw, g0);
+        asm volatile("" ::: "memory");
+        copy_item(g0, 0, slot0);
+        copy_item(kMG == 1 ? min(g0 + 1, g1 - 1) : g0, kMG == 1 ? 0 : 1, slot1);
+        // Group g, its first item in slot `par`.  Loads past the slice's end re-read its last
+        // group (cache hits) and are never consumed.
+        auto group = [&](int g, int par) {
+            fence();
+            Ops O;
+            convert(O, raw);
+            fence();
+            load_raw(raw, min(g + 1, g1 - 1));
+            fence();
+#pragma unroll
+            for (int mg = 0; mg < kMG; ++mg) {  // the item two ahead: group g + (mg + 2) / kMG
+                const int ng = g + (mg + 2) / kMG;
+                item(O, mg, (par + mg) & 1 ? slot1 : slot0, kMG == 1 ? 2 : mg < 2 ? 1 : 0, min(ng, g1 - 1),
+                     (mg + 2) % kMG);
+            }
+        };
+        if constexpr (kMG == 1) {
+            int g = g0;
+            for (; g + 1 < g1; g += 2) {
+                group(g, 0);
+                group(g + 1, 1);
+            }
+            if (g < g1) group(g, 0);
+        } else {
+            for (int g = g0; g < g1; ++g) group(g, 0);
+        }
+        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // no copy may land after the slots are reused
+    }
+
+    // The W K slices of each row group meet in LDS and are added in wave order (eight
+    // waves: each half in wave order, then the two halves).
+#pragma unroll
+    for (int mg = 0; mg < kMG; ++mg) {
+        float* lds = reinterpret_cast<float*>(mg & 1 ? slot1 : slot0);
+        if (mg == 0) __syncthreads();  // every wave is done with its slots
+#pragma unroll
+        for (int i = 0; i < kNT; ++i)
+            *reinterpret_cast<f32x4*>(lds + ((wave * kNT + i) * 64 + lane) * 4) = acc[mg][i];
+        __syncthreads();
+        for (int f = (int)threadIdx.x; f < kRH * T * 256; f += 64 * W * kRH) {
+            const int h = f / (T * 256), i = (f >> 8) % T, b = (f >> 4) & 15, r = f & 15;
+            const int row = (tile0 + i) * kTileRows + r, br = (h * kMG + mg) * 16 + b;
+            if (br >= batch || tile0 + i >= n_tiles || row >= n_rows) continue;
+            const int src = h * W * kNT * 256 + ((b >> 2) * 16 + r) * 4 + (b & 3);
+            float v[kNW];
+#pragma unroll
+            for (int nw = 0; nw < kNW; ++nw) {
+                v[nw] = lds[(nw * T + i) * 256 + src];
+#pragma unroll
+                for (int w = 1; w < kWH; ++w) v[nw] += lds[((w * kNT) + nw * T + i) * 256 + src];
+                if constexpr (W == 8) {
+                    float e = lds[((4 * kNT) + nw * T + i) * 256 + src];
+#pragma unroll
+                    for (int w = 5; w < 8; ++w) e += lds[((w * kNT) + nw * T + i) * 256 + src];
+                    v[nw] += e;
+                }
+            }
+            if constexpr (kNW == 2)
+                y[(size_t)br * n_rows + row] = v[0] / (1.0f + expf(-v[0])) * v[1];
+            else
+                y[(size_t)br * n_rows + row] = v[0];
+        }
+    }
+}
+
 template <int kFmt, int T, int W, int kNW, int kRep>
 hipError_t run(const Weight& w, const uint8_t* w1, const float* x, float* y, int batch, int splits,
                hipStream_t s) {
@@ -555,20 +935,104 @@ hipError_t run(const Weight& w, const uint8_t* w1, const float* x, float* y, int
     return hipGetLastError();
 }
 
+template <int kFmt, int T, int W, int kNW, int kRH, int kMG>
+hipError_t run_rows(const Weight& w, const uint8_t* w1, const float* x, float* y, int batch, hipStream_t s) {
+    const unsigned wgs = (unsigned)((w.n_tiles + T - 1) / T);
+    hipLaunchKernelGGL((gemv_rows_kernel<kFmt, T, W, kNW, kRH, kMG>), dim3(wgs), dim3(64 * W * kRH), 0, s, w.chunks, w1, x, y,
+                       (int)w.n, (int)w.n_tiles, (int)w.groups, (int)w.k, batch);
+    return hipGetLastError();
+}
+
 }  // namespace
+
+constexpr int64_t kCUs = 256;  // MI355X compute units
 
 bool use_batch_kernel(const Weight& w, int64_t batch) {
     return batch >= kBatchMin && (int64_t)kBatchRows * w.k * 4 <= INT32_MAX;
 }
 
+// The multi-row-group launch of a weight (or pair): T row tiles and W K slices per
+// workgroup.  The waves cut K as a 16-row call's do, so a row has the same bits in either:
+// its own wave count, or eight slices in place of a two-way split over four-wave
+// workgroups (gemv_batch_kernel's halves).  Splits with more waves than that, and K of
+// fewer than 8 groups (one wave), have no such form and stay on 16-row passes (w = 0).  So do
+// weights of more than 768 row tiles: one pass holds at most 3 tiles per workgroup, 16-row
+// passes up to 8, and the activation split is shared by fewer tiles than the saved passes
+// win back (28672 x 8192, 20 / 40 rows: 75 / 109 us against 63 / 98); a pair, at one tile of
+// each weight, from 512 on (11008 x 4096, 20 / 40 rows: 39.7 / 51.4 us against 32.3 / 50.3).
+constexpr int kRowsMax = 4 * kBatchRows;  // rows of one multi-row-group launch
+struct RowsShape {
+    int t = 1, w = 0;
+};
+static RowsShape choose_rows_shape(const Weight& w, bool pair) {
+    const BatchShape sh = choose_batch_shape(w, kBatchRows, pair);
+    RowsShape r;
+    const int64_t per_cu = (w.n_tiles + kCUs - 1) / kCUs;
+    if (per_cu > (pair ? 2 : 3)) return r;
+    if (sh.split == 1 && sh.w >= 4)
+        r.w = sh.w;
+    else if (sh.split == 2 && sh.w == 4)
+        r.w = 8;
+    r.t = pair ? 1 : (int)per_cu;
+    return r;
+}
+
+// Four K slices run two row halves of waves (kGroups / 2 row groups each), eight one.
+template <int kFmt, int kGroups>
+static hipError_t dispatch_rows(const Weight& w, const Weight* up, const float* x, float* y, int batch,
+                                const RowsShape& sh, hipStream_t s) {
+    if (up) return sh.w == 4 ? run_rows<kFmt, 1, 4, 2, 2, kGroups / 2>(w, up->chunks, x, y, batch, s) : hipErrorInvalidValue;
+#define QMM_ROWS_CASE(T_)                                                                             \
+    if (sh.t == T_)                                                                                   \
+        return sh.w == 8 ? run_rows<kFmt, T_, 8, 1, 1, kGroups>(w, nullptr, x, y, batch, s)           \
+                         : run_rows<kFmt, T_, 4, 1, 2, kGroups / 2>(w, nullptr, x, y, batch, s);
+    QMM_ROWS_CASE(1)
+    QMM_ROWS_CASE(2)
+    QMM_ROWS_CASE(3)
+#undef QMM_ROWS_CASE
+    return hipErrorInvalidValue;
+}
+
+template <int kFmt>
+static hipError_t dispatch_groups(const Weight& w, const Weight* up, const float* x, float* y, int batch,
+                                  const RowsShape& sh, hipStream_t s) {
+    return batch <= 2 * kBatchRows ? dispatch_rows<kFmt, 2>(w, up, x, y, batch, sh, s)
+                                   : dispatch_rows<kFmt, 4>(w, up, x, y, batch, sh, s);
+}
+
+// y[batch][n] for 17 .. kRowsMax rows in one pass over W.
+static hipError_t launch_rows(const Weight& w, const Weight* up, const float* x, float* y, int batch,
+                              const RowsShape& sh, hipStream_t s) {
+    switch (w.type) {
+    case OPENMINI_QMM_Q4_0: return dispatch_groups<OPENMINI_QMM_Q4_0>(w, up, x, y, batch, sh, s);
+    case OPENMINI_QMM_Q8_0: return dispatch_groups<OPENMINI_QMM_Q8_0>(w, up, x, y, batch, sh, s);
+    case OPENMINI_QMM_Q4_K: return dispatch_groups<OPENMINI_QMM_Q4_K>(w, up, x, y, batch, sh, s);
+    case OPENMINI_QMM_Q6_K: return dispatch_groups<OPENMINI_QMM_Q6_K>(w, up, x, y, batch, sh, s);
+    case OPENMINI_QMM_Q4_1: return dispatch_groups<OPENMINI_QMM_Q4_1>(w, up, x, y, batch, sh, s);
+    case OPENMINI_QMM_Q5_K: return dispatch_groups<OPENMINI_QMM_Q5_K>(w, up, x, y, batch, sh, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_gemv_rows(const Weight& w, const Weight* up, const float* x, float* y, int64_t batch,
                             hipStream_t s) {
     if (use_batch_kernel(w, batch)) {
-        for (int64_t b0 = 0; b0 < batch; b0 += kBatchRows) {
-            const int nb = (int)(batch - b0 < kBatchRows ? batch - b0 : kBatchRows);
-            const hipError_t e =
-                launch_gemv_batch(w, up, x + b0 * w.k, y + b0 * w.n, nb, choose_batch_shape(w, nb, up), s);
+        const RowsShape rows = choose_rows_shape(w, up != nullptr);
+        // A pair holds two weights' operands per tile, so one tile per workgroup: that pays
+        // from three row groups on (Q5_K 8192 x 4096, 20 / 40 rows: 36.9 -> 39.8, 58.3 -> 49.9 us).
+        const int64_t least = up ? 2 * kBatchRows : kBatchRows;
+        const bool multi = rows.w != 0 && (int64_t)kRowsMax * w.k * 4 <= INT32_MAX;  // 31-bit x offsets
+        for (int64_t b0 = 0; b0 < batch;) {
+            const int64_t rest = batch - b0;
+            const bool many = multi && rest > least;
+            const int64_t most = many ? kRowsMax : kBatchRows;
+            const int nb = (int)(rest < most ? rest : most);
+            const float* xs = x + b0 * w.k;
+            float* ys = y + b0 * w.n;
+            const hipError_t e = many ? launch_rows(w, up, xs, ys, nb, rows, s)
+                                      : launch_gemv_batch(w, up, xs, ys, nb, choose_batch_shape(w, nb, up), s);
             if (e != hipSuccess) return e;
+            b0 += nb;
         }
         return hipSuccess;
     }
@@ -597,8 +1061,6 @@ hipError_t launch_gemv_rows(const Weight& w, const Weight* up, const float* x, f
 // vs 8: 45.4 vs 47.8 us.  A (gate, up) pair takes at most 4 (Q4_0 / Q4_K) or 3 tiles:
 // against one tile per workgroup, 11008 x 4096 Q4_0 B = 8 25.5 -> 20.8 us, Q8_0 B = 8
 // 30.7 -> 25.2 us, Q4_K B = 16 31.9 -> 22.5 us, 28672 x 8192 Q4_0 B = 16 118 -> 80 us.
-constexpr int64_t kCUs = 256;  // MI355X compute units
-
 static int64_t tiles_per_cu(int type, int64_t n_tiles, bool pair) {
     // a pair holds two weights' registers per tile: at most 4 / 3 tiles
     const bool nib = type == OPENMINI_QMM_Q4_0 || type == OPENMINI_QMM_Q4_K || type == OPENMINI_QMM_Q4_1;

@@ -322,3 +322,60 @@ def test_batch_linearity_full_size(qmm):
     p = assert_parity(y12, 2.0 * y1.astype(np.float64) + y2, TOL, "linearity")
     assert p["normwise"] <= 2e-6, p
     assert np.all(run_gemv(qmm, w, np.zeros((16, K), np.float32)) == 0.0)
+
+
+def run_pair(qmm, gate, up, x):
+    B = x.shape[0]
+    dx = qmm.DeviceBuffer.from_numpy(np.ascontiguousarray(x))
+    dh = qmm.DeviceBuffer(B * gate.n_rows * 4)
+    qmm.ffn_gate_up(gate, up, dx, dh, B)
+    return dh.download(np.float32, (B, gate.n_rows))
+
+
+@pytest.mark.parametrize("qtype", [Q4_0, 3, Q8_0, 12, 13, 14])
+@pytest.mark.parametrize("N,K,B", [
+    (40, 1024, 17), (777, 2304, 33),      # tiles past the weight; a row group of one row
+    (1000, 4096, 47), (4100, 4096, 32),   # a K split's halves as eight slices; two tiles per workgroup
+    (8200, 1280, 64), (4096, 8192, 80)])  # three tiles; two launches
+def test_many_rows_equal_16_row_calls(qmm, orc, qtype, N, K, B):
+    """17 to 64 rows go through the weight in one pass: each row's result is bit for bit
+    that of a 16-row call on it (and within the contract's tolerance of fp64), single
+    weights and (gate, up) pairs."""
+    def blocks(seed):
+        return (synth.kquant_blocks(qtype, N, K, seed=seed) if qtype in (12, 13, 14)
+                else synth.weight_blocks(qtype, N, K, seed=seed))
+    x = synth.normal(0xBA1 + B, (B, K), 1.0)
+    b0, b1 = blocks(0xBA2 + N), blocks(0xBA3 + N)
+    w, up = qmm.QuantizedWeight(qtype, b0, N, K), qmm.QuantizedWeight(qtype, b1, N, K)
+    print(f"many rows type={qtype} N={N} K={K} B={B}", flush=True)
+    y = run_gemv(qmm, w, x)
+    h = run_pair(qmm, w, up, x)
+    for lo in range(0, B, 16):
+        hi = min(B, lo + 16)
+        if hi - lo < 4:  # fewer rows than the batched kernel takes: with three more before them
+            lo = hi - 4
+        assert np.array_equal(y[lo:hi].view(np.uint32), run_gemv(qmm, w, x[lo:hi]).view(np.uint32)), (lo, hi)
+        assert np.array_equal(h[lo:hi].view(np.uint32), run_pair(qmm, w, up, x[lo:hi]).view(np.uint32)), (lo, hi)
+    rows = [0, 15, 16, B - 1]
+    assert_parity(y[rows], orc.linear_f64(qtype, b0, N, K, x[rows]), TOL, f"{qtype} {N}x{K} B={B}")
+
+
+def test_many_rows_nonfinite_and_ragged(qmm):
+    """Rows holding inf / NaN keep to themselves across row groups, and a last K group of
+    fewer than 4 blocks reads nothing past a row (x ends in a NaN tail)."""
+    N, K, B = 300, 1120, 40
+    w = qmm.QuantizedWeight(Q8_0, synth.weight_blocks(Q8_0, N, K, seed=0xBB0), N, K)
+    x = synth.normal(0xBB1, (B, K), 1.0)
+    clean = run_gemv(qmm, w, x)
+    bad = x.copy()
+    bad[3, 7], bad[20, K - 1], bad[33, 500] = np.inf, np.nan, -np.inf
+    y = run_gemv(qmm, w, bad)
+    ok = [r for r in range(B) if r not in (3, 20, 33)]
+    assert np.array_equal(y[ok].view(np.uint32), clean[ok].view(np.uint32))
+    assert not np.any(np.isfinite(y[[3, 20, 33]]))
+    dx = qmm.DeviceBuffer((B + 2) * K * 4)
+    dx.fill(0xFF)
+    dx.upload(x)
+    dy = qmm.DeviceBuffer(B * N * 4)
+    w.gemv(dx, dy, B)
+    assert np.array_equal(dy.download(np.float32, (B, N)).view(np.uint32), clean.view(np.uint32))
