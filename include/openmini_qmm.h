@@ -243,9 +243,9 @@ int openmini_qmm_gemm_f32(const openmini_qweight_t* weight, const float* d_x, fl
 /* ---- projections of one layer (src/model/inference/model.rs) ----------------------- */
 
 /* Weights that share the input: d_ys[i][batch, N_i] = x[batch, K] . W_i^T for
- * i < count (1..4), all of one type and one K; one launch for up to 3 batch rows,
- * or from 4 rows on one batched pass per weight (results identical to
- * openmini_qmm_gemv of each weight).  Replaces the three linear_gemm calls of prepare_qkv
+ * i < count (1..4), all of one type and one K; one launch for up to 3 batch rows and,
+ * for weights that together fill the chip once, for 4 to 16, else one batched pass per
+ * weight (results identical to openmini_qmm_gemv of each weight).  Replaces the three linear_gemm calls of prepare_qkv
  * (model.rs:1392-1394: q, k, v of one normalised hidden state).  d_x must be
  * 16-byte aligned. */
 int openmini_qmm_gemv_multi(const openmini_qweight_t* const* weights, int count, const float* d_x,

@@ -591,7 +591,12 @@ int openmini_qmm_gemv_multi(const openmini_qweight_t* const* weights, int count,
     if (tiles > INT32_MAX) return fail(OPENMINI_QMM_ERR_INVALID_PARAM, "too many rows in one group");
     const int64_t k = ws[0]->k;
     if (qmm::use_batch_kernel(*ws[0], batch)) {
-        // several rows: one batched pass per weight
+        // several rows: one batched launch for all weights where that is faster, else per weight
+        if (qmm::use_batch_group(ws, count, batch)) {
+            hipError_t e = qmm::launch_gemv_batch_group(ws, d_ys, count, d_x, (int)batch, as_stream(stream));
+            if (e != hipSuccess) return hip_fail(e, "gemv_multi launch");
+            return ok();
+        }
         for (int i = 0; i < count; ++i) {
             hipError_t e = qmm::launch_gemv_rows(*ws[i], nullptr, d_x, d_ys[i], batch, as_stream(stream));
             if (e != hipSuccess) return hip_fail(e, "gemv_multi launch");

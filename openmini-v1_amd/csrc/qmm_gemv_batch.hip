@@ -190,12 +190,10 @@ __device__ __forceinline__ f16x8 codes_q5(uint32_t w, uint32_t qh) {
 // stored), and every stored result follows the same arithmetic whatever kRep (bitwise
 // identical for any batch size).
 template <int kFmt, int T, int W, int kNW, int kRep>
-__global__ __launch_bounds__(64 * W) void gemv_batch_kernel(const uint8_t* __restrict__ w0,
-                                                            const uint8_t* __restrict__ w1,
-                                                            const float* __restrict__ x, float* __restrict__ y,
-                                                            int n_rows, int n_tiles, int groups, int k, int batch,
-                                                            float* __restrict__ sums, uint32_t* __restrict__ cnt,
-                                                            int splits) {
+__device__ __forceinline__ void gemv_batch_body(const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1,
+                                                const float* __restrict__ x, float* __restrict__ y, int n_rows,
+                                                int n_tiles, int groups, int k, int batch, float* __restrict__ sums,
+                                                uint32_t* __restrict__ cnt, int splits, int block) {
     static_assert(kRep == 1 || kRep == 2 || kRep == 4, "lanes per activation row");
     constexpr int kNT = kNW * T;  // (weight, tile) pairs of the workgroup
     constexpr int kXB = 4 / kRep;  // blocks of a group a lane loads and splits
@@ -216,8 +214,8 @@ __global__ __launch_bounds__(64 * W) void gemv_batch_kernel(const uint8_t* __res
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, kq = lane >> 4;
     // workgroup = (tile group, K split): the split's contiguous K groups [gs0, gs1)
-    const int split = (int)blockIdx.x % splits;
-    const int tgroup = (int)blockIdx.x / splits;
+    const int split = block % splits;
+    const int tgroup = block / splits;
     const int tile0 = tgroup * T;
     const int gs0 = (int)((int64_t)groups * split / splits);
     const int gsn = (int)((int64_t)groups * (split + 1) / splits) - gs0;
@@ -545,6 +543,38 @@ __global__ __launch_bounds__(64 * W) void gemv_batch_kernel(const uint8_t* __res
             y[(size_t)b * n_rows + row] = v;
         }
     }
+}
+
+template <int kFmt, int T, int W, int kNW, int kRep>
+__global__ __launch_bounds__(64 * W) void gemv_batch_kernel(const uint8_t* __restrict__ w0,
+                                                            const uint8_t* __restrict__ w1,
+                                                            const float* __restrict__ x, float* __restrict__ y,
+                                                            int n_rows, int n_tiles, int groups, int k, int batch,
+                                                            float* __restrict__ sums, uint32_t* __restrict__ cnt,
+                                                            int splits) {
+    gemv_batch_body<kFmt, T, W, kNW, kRep>(w0, w1, x, y, n_rows, n_tiles, groups, k, batch, sums, cnt, splits,
+                                           (int)blockIdx.x);
+}
+
+// Several weights of one type and K on the same activations (q / k / v), one launch: a
+// workgroup takes T tiles of one of them, eight waves over all of K -- the cut and the
+// addition order of a two-way K split, so each output has the bits of its weight's own
+// call, without the split's hand-off.
+struct BatchGroup {
+    int begin[kMaxGroup + 1];  // weight g's workgroups; entries past the last weight hold the grid size
+    int n_rows[kMaxGroup], n_tiles[kMaxGroup];
+    const uint8_t* chunks[kMaxGroup];
+    float* y[kMaxGroup];
+};
+
+template <int kFmt, int T, int kRep>
+__global__ __launch_bounds__(512) void gemv_batch_group_kernel(const float* __restrict__ x, int groups, int k, int batch,
+                                                               const BatchGroup grp) {
+    int g = 0;  // uniform
+#pragma unroll
+    for (int i = 1; i < kMaxGroup; ++i) g += (int)blockIdx.x >= grp.begin[i] ? 1 : 0;
+    gemv_batch_body<kFmt, T, 8, 1, kRep>(grp.chunks[g], nullptr, x, grp.y[g], grp.n_rows[g], grp.n_tiles[g], groups, k,
+                                         batch, nullptr, nullptr, 1, (int)blockIdx.x - grp.begin[g]);
 }
 
 // A K group's weights of kNT (weight, tile) pairs as loaded: chunk slot `lane` whole.
@@ -1206,6 +1236,87 @@ hipError_t launch_gemv_batch(const Weight& w, const Weight* up, const float* x, 
     case OPENMINI_QMM_Q5_K:
         return up ? dispatch_rep<OPENMINI_QMM_Q5_K, 2>(w, w1, x, y, batch, sh, s)
                   : dispatch_rep<OPENMINI_QMM_Q5_K, 1>(w, w1, x, y, batch, sh, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+template <int kFmt, int kRep>
+static hipError_t dispatch_batch_group(const BatchGroup& grp, const Weight& w, const float* x, int batch, int t,
+                                       hipStream_t s) {
+    const dim3 grid((unsigned)grp.begin[kMaxGroup]);
+    const int groups = (int)w.groups, k = (int)w.k;
+#define QMM_GROUP_CASE(T_)                                                                                       \
+    case T_:                                                                                                     \
+        hipLaunchKernelGGL((gemv_batch_group_kernel<kFmt, T_, kRep>), grid, dim3(512), 0, s, x, groups, k, batch, grp); \
+        return hipGetLastError();
+    switch (t) {
+        QMM_GROUP_CASE(1)
+        QMM_GROUP_CASE(2)
+        QMM_GROUP_CASE(3)
+        QMM_GROUP_CASE(4)
+    default: return hipErrorInvalidValue;
+    }
+#undef QMM_GROUP_CASE
+}
+
+template <int kFmt>
+static hipError_t dispatch_batch_group_rep(const BatchGroup& grp, const Weight& w, const float* x, int batch, int t,
+                                           hipStream_t s) {
+    if (batch <= 4) return dispatch_batch_group<kFmt, 4>(grp, w, x, batch, t, s);
+    if (batch <= 8) return dispatch_batch_group<kFmt, 2>(grp, w, x, batch, t, s);
+    return dispatch_batch_group<kFmt, 1>(grp, w, x, batch, t, s);
+}
+
+// Tiles per workgroup of a projection group's one launch, 0 for separate launches.  A weight
+// that alone would run a two-way K split (or its eight-wave form) holds at most 512 tiles: at
+// most one workgroup per CU works on 2 to 4 of them, and the activation split is done over
+// again for every weight.  Together they take the fewest tiles per workgroup, up to 4, with
+// which the whole group is one workgroup per CU: two workgroups over that are a second round
+// (three Q8_0 4096 x 4096, 8 rows: 20.7 us with 3 tiles in 258 workgroups, 14.2 with 4 in 192;
+// 22.7 in separate launches).  Others, 8 rows, separate -> one launch: Q4_K 4096 + 2 x 1024
+// rows x 4096 19.4 -> 8.6 us, Q6_K 3 x 5120 x 5120 45.0 -> 22.2.  More tiles fill the chip one
+// weight at a time.
+static int batch_group_tiles(const Weight* const* ws, int count) {
+    for (int i = 0; i < count; ++i) {
+        const BatchShape sh = choose_batch_shape(*ws[i], kBatchRows, false);
+        if (!(sh.split == 2 && sh.w == 4) && !(sh.split == 1 && sh.w == 8)) return 0;
+    }
+    for (int t = 1; t <= 4; ++t) {
+        int64_t wgs = 0;
+        for (int i = 0; i < count; ++i) wgs += (ws[i]->n_tiles + t - 1) / t;
+        if (wgs <= kCUs) return t;
+    }
+    return 0;
+}
+
+bool use_batch_group(const Weight* const* ws, int count, int64_t batch) {
+    return count >= 2 && count <= kMaxGroup && batch <= kBatchRows && use_batch_kernel(*ws[0], batch) &&
+           batch_group_tiles(ws, count) > 0;
+}
+
+hipError_t launch_gemv_batch_group(const Weight* const* ws, float* const* ys, int count, const float* x, int batch,
+                                   hipStream_t s) {
+    if (!use_batch_group(ws, count, batch)) return hipErrorInvalidValue;
+    const int t = batch_group_tiles(ws, count);
+    BatchGroup grp{};
+    int64_t wgs = 0;
+    for (int i = 0; i < count; ++i) {
+        grp.begin[i] = (int)wgs;
+        grp.n_rows[i] = (int)ws[i]->n;
+        grp.n_tiles[i] = (int)ws[i]->n_tiles;
+        grp.chunks[i] = ws[i]->chunks;
+        grp.y[i] = ys[i];
+        wgs += (ws[i]->n_tiles + t - 1) / t;
+    }
+    for (int i = count; i <= kMaxGroup; ++i) grp.begin[i] = (int)wgs;
+    const Weight& w = *ws[0];
+    switch (w.type) {
+    case OPENMINI_QMM_Q4_0: return dispatch_batch_group_rep<OPENMINI_QMM_Q4_0>(grp, w, x, batch, t, s);
+    case OPENMINI_QMM_Q8_0: return dispatch_batch_group_rep<OPENMINI_QMM_Q8_0>(grp, w, x, batch, t, s);
+    case OPENMINI_QMM_Q4_K: return dispatch_batch_group_rep<OPENMINI_QMM_Q4_K>(grp, w, x, batch, t, s);
+    case OPENMINI_QMM_Q6_K: return dispatch_batch_group_rep<OPENMINI_QMM_Q6_K>(grp, w, x, batch, t, s);
+    case OPENMINI_QMM_Q4_1: return dispatch_batch_group_rep<OPENMINI_QMM_Q4_1>(grp, w, x, batch, t, s);
+    case OPENMINI_QMM_Q5_K: return dispatch_batch_group_rep<OPENMINI_QMM_Q5_K>(grp, w, x, batch, t, s);
     default: return hipErrorInvalidValue;
     }
 }

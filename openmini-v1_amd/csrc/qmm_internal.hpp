@@ -275,6 +275,12 @@ size_t split_workspace_bytes(int64_t n_tiles, int t, int s);
 hipError_t launch_gemv_batch(const Weight& w, const Weight* up, const float* x, float* y, int batch,
                              const BatchShape& sh, hipStream_t s);
 
+// ys[i][batch][n_i] = x . W_i^T for weights of one type and K in one launch, where
+// use_batch_group says so (4 .. kBatchRows rows); the bits are those of each weight's own call.
+bool use_batch_group(const Weight* const* ws, int count, int64_t batch);
+hipError_t launch_gemv_batch_group(const Weight* const* ws, float* const* ys, int count, const float* x, int batch,
+                                   hipStream_t s);
+
 // y[m][n] = x_bf16[m][k] . W^T.
 // gate_in_y: y holds gate = x . Wg^T on entry; each element becomes silu(gate) * (x . W^T).
 hipError_t launch_gemm_bf16(const Weight& w, const uint16_t* x, float* y, int64_t m, hipStream_t s,

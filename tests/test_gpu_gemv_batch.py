@@ -379,3 +379,27 @@ def test_many_rows_nonfinite_and_ragged(qmm):
     dy = qmm.DeviceBuffer(B * N * 4)
     w.gemv(dx, dy, B)
     assert np.array_equal(dy.download(np.float32, (B, N)).view(np.uint32), clean.view(np.uint32))
+
+
+@pytest.mark.parametrize("qtype", [Q4_0, 3, Q8_0, 12, 13, 14])
+@pytest.mark.parametrize("Ns,K,B", [
+    ((4096, 1024, 1024), 4096, 8),             # grouped: two tiles per workgroup
+    ((2100, 4000, 37, 5), 4096, 4),            # four weights, ragged row counts
+    ((5120, 5120, 5120), 4096, 16),            # four tiles
+    ((4096, 4096, 8200), 4096, 5),             # one weight does not split: separate launches
+    ((1024, 700), 8192, 9)])                   # four-way splits: separate launches
+def test_multi_equals_single_calls(qmm, qtype, Ns, K, B):
+    """gemv_multi of several rows gives each weight's own call bit for bit, in one launch
+    or in several."""
+    ws = [qmm.QuantizedWeight(qtype, (synth.kquant_blocks(qtype, n, K, seed=0xBC0 + i) if qtype in (12, 13, 14)
+                                      else synth.weight_blocks(qtype, n, K, seed=0xBC0 + i)), n, K)
+          for i, n in enumerate(Ns)]
+    x = synth.normal(0xBC9, (B, K), 1.0)
+    dx = qmm.DeviceBuffer.from_numpy(x)
+    dys = [qmm.DeviceBuffer(B * n * 4) for n in Ns]
+    for d in dys:
+        d.fill(0xFF)
+    print(f"gemv_multi type={qtype} N={Ns} K={K} B={B}", flush=True)
+    qmm.gemv_multi(ws, dx, dys, B)
+    for w, d, n in zip(ws, dys, Ns):
+        assert np.array_equal(d.download(np.uint32, (B, n)), run_gemv(qmm, w, x).view(np.uint32)), n
