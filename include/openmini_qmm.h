@@ -274,8 +274,10 @@ int openmini_qmm_ffn_gate_up_f32(const openmini_qweight_t* gate, const openmini_
 /* GemmEngine::matmul-shaped convenience on host memory: y[m, N] = x[m, K] . W^T,
  * fp32 in/out, synchronous.  Below openmini_qmm_gemm_min_rows rows (64-128, by the
  * weight's shape) the decode GEMVs, from there on the fp32 prefill GEMM
- * (openmini_qmm_gemm_f32; Q4_1 / Q5_K weights: the batched GEMV at any row count); x,
- * y and the GEMM's workspace are allocated per call. */
+ * (openmini_qmm_gemm_f32; Q4_1 / Q5_K weights: the batched GEMV at any row count).
+ * x, y and the GEMM's workspace are staged through the 16 MiB array of
+ * openmini_qmm_linear_host_noalloc where they fit and no other call holds it, else
+ * allocated per call. */
 int openmini_qmm_linear_host(const openmini_qweight_t* weight, const float* x, float* y,
                              int64_t m);
 

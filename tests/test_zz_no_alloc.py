@@ -120,6 +120,43 @@ def test_noalloc_concurrent_threads(qmm):
     assert not errors, errors
 
 
+def test_linear_host_staged_or_allocated(qmm):
+    """linear_host takes the staging array while it is free and allocates otherwise: four
+    threads at once on one weight and on their own, among them calls past the array's
+    size and calls of linear_host_noalloc, give the bits of device buffers of their own."""
+    import threading
+    L = _native.lib()
+    shared = qmm.QuantizedWeight(Q4_0, synth.weight_blocks(Q4_0, 4096, 4096, seed=0xA70), 4096, 4096)
+    small = qmm.QuantizedWeight(Q8_0, synth.weight_blocks(Q8_0, 1000, 2080, seed=0xA71), 1000, 2080)
+    calls = [(shared, 1, L.openmini_qmm_linear_host), (shared, 9, L.openmini_qmm_linear_host),
+             (shared, 600, L.openmini_qmm_linear_host), (small, 3, L.openmini_qmm_linear_host_noalloc)]
+    work = []
+    for i, (w, m, call) in enumerate(calls):
+        x = synth.normal(0xA72 + i, (m, w.k_cols), 1.0)
+        dx, dy = qmm.DeviceBuffer.from_numpy(x), qmm.DeviceBuffer(m * w.n_rows * 4)
+        if m >= w.gemm_min_rows():
+            w.gemm_f32(dx, dy, m, qmm.gemm_f32_workspace(m, w.k_cols))
+        else:
+            w.gemv(dx, dy, m)
+        work.append((w, call, x, dy.download(np.uint32, (m, w.n_rows))))
+    errors = []
+
+    def run(w, call, x, ref):
+        for r in range(8):
+            y = np.full(ref.shape, np.nan, np.float32)
+            rc = call(w.handle, _ptr(x), _ptr(y), x.shape[0])
+            if rc != 0 or not np.array_equal(y.view(np.uint32), ref):
+                errors.append((x.shape, r, rc))
+
+    print("linear_host: 4 threads x 8 calls", flush=True)
+    threads = [threading.Thread(target=run, args=a) for a in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+
+
 def test_noalloc_leaves_device_memory_unchanged(qmm):
     """After a warm-up call, further calls leave the device's free memory where it
     was (hipMemGetInfo): the staging array is static, nothing is allocated or kept."""
