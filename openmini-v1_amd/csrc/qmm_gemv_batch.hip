@@ -56,6 +56,7 @@
 // itself in; the last to arrive adds the splits' sums in split order, so the result
 // does not depend on which one finishes last.
 #include "qmm_device.hpp"
+#include "qmm_rows_walk.hpp"
 
 namespace qmm {
 namespace {
@@ -620,7 +621,6 @@ __global__ __launch_bounds__(64 * W * kRH, 2) void gemv_rows_kernel(const uint8_
                                                               const uint8_t* __restrict__ w1,
                                                               const float* __restrict__ x, float* __restrict__ y,
                                                               int n_rows, int n_tiles, int groups, int k, int batch) {
-    static_assert(kMG == 1 || kMG % 2 == 0, "the items of a K group start in slot 0, or alternate");
     constexpr int kNT = kNW * T;
     using F = BFmt<kFmt>;
     constexpr int kCB = F::kCB;
@@ -718,6 +718,21 @@ __global__ __launch_bounds__(64 * W * kRH, 2) void gemv_rows_kernel(const uint8_
         }
     };
 
+    // Counts as a use of every load of R.
+    auto keep = [](const Raw& R) {
+#pragma unroll
+        for (int i = 0; i < kNT; ++i) {
+#pragma unroll
+            for (int h = 0; h < (F::kQ8 ? 2 : 1); ++h)
+                asm volatile("" ::"v"(R.c[i][h].x), "v"(R.c[i][h].y), "v"(R.c[i][h].z), "v"(R.c[i][h].w));
+            asm volatile("" ::"v"(R.sc[i]));
+            if constexpr (F::kQ6K) asm volatile("" ::"v"(R.hb[i].x));
+            if constexpr (F::kKQ) asm volatile("" ::"v"(R.dk[i]));
+            if constexpr (F::kMin) asm volatile("" ::"v"(R.mn[i]));
+            if constexpr (F::kQ5) asm volatile("" ::"v"(R.dm[i]));
+        }
+    };
+
     auto convert = [&](Ops& O, const Raw& R) {
 #pragma unroll
         for (int i = 0; i < kNT; ++i) {
@@ -786,13 +801,13 @@ __global__ __launch_bounds__(64 * W * kRH, 2) void gemv_rows_kernel(const uint8_
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto item = [&](const Ops& O, int mg, uint8_t* slot, int ahead, int next_g, int next_mg) {
+    auto item = [&](const Ops& O, int mg, uint8_t* slot, int raws, int next_g, int next_mg) {
         fence();
         // this item's copies have landed: at most the loads issued after them -- the next
-        // item's copies and `ahead` groups' weights -- are out
-        if (ahead == 0)
+        // item's copies and `raws` groups' weights (walk_rows) -- are out
+        if (raws == 0)
             __builtin_amdgcn_s_waitcnt(vmcnt_only(kCopies));
-        else if (ahead == 1)
+        else if (raws == 1)
             __builtin_amdgcn_s_waitcnt(vmcnt_only(kCopies + kRawLoads));
         else
             __builtin_amdgcn_s_waitcnt(vmcnt_only(kCopies + 2 * kRawLoads));
@@ -886,37 +901,27 @@ __global__ __launch_bounds__(64 * W * kRH, 2) void gemv_rows_kernel(const uint8_
 
     if (g0 < g1 && wrows > 0) {  // uniform per wave
         Raw raw;
-        load_raw(raw, g0);
-        asm volatile("" ::: "memory");
-        copy_item(g0, 0, slot0);
-        copy_item(kMG == 1 ? min(g0 + 1, g1 - 1) : g0, kMG == 1 ? 0 : 1, slot1);
-        // Group g, its first item in slot `par`.  Loads past the slice's end re-read its last
-        // group (cache hits) and are never consumed.
-        auto group = [&](int g, int par) {
-            fence();
-            Ops O;
-            convert(O, raw);
-            fence();
-            load_raw(raw, min(g + 1, g1 - 1));
-            fence();
-#pragma unroll
-            for (int mg = 0; mg < kMG; ++mg) {  // the item two ahead: group g + (mg + 2) / kMG
-                const int ng = g + (mg + 2) / kMG;
-                item(O, mg, (par + mg) & 1 ? slot1 : slot0, kMG == 1 ? 2 : mg < 2 ? 1 : 0, min(ng, g1 - 1),
-                     (mg + 2) % kMG);
-            }
-        };
-        if constexpr (kMG == 1) {
-            int g = g0;
-            for (; g + 1 < g1; g += 2) {
-                group(g, 0);
-                group(g + 1, 1);
-            }
-            if (g < g1) group(g, 0);
-        } else {
-            for (int g = g0; g < g1; ++g) group(g, 0);
-        }
-        __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // no copy may land after the slots are reused
+        Ops O;
+        walk_rows<kMG>(
+            g0, g1,
+            [&](int g) {
+                fence();
+                load_raw(raw, g);
+                fence();
+            },
+            [&] {
+                fence();
+                convert(O, raw);
+                fence();
+            },
+            [&](int g, int mg, int slot) { copy_item(g, mg, slot ? slot1 : slot0); },
+            [&](int mg, int slot, int raws, int next_g, int next_mg) {
+                item(O, mg, slot ? slot1 : slot0, raws, next_g, next_mg);
+            },
+            [&] {
+                keep(raw);
+                __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // no copy may land after the slots are reused
+            });
     }
 
     // The W K slices of each row group meet in LDS and are added in wave order (eight
