@@ -56,6 +56,7 @@
 // itself in; the last to arrive adds the splits' sums in split order, so the result
 // does not depend on which one finishes last.
 #include "qmm_device.hpp"
+#include "qmm_rows_shape.hpp"
 #include "qmm_rows_walk.hpp"
 
 namespace qmm {
@@ -627,6 +628,10 @@ __global__ __launch_bounds__(64 * W * kRH, 2) void gemv_rows_kernel(const uint8_
     constexpr int kCodeBytes = kTileEntries * kCB;
     constexpr int kChunk = F::kChunk;
     constexpr bool kQ6 = F::kQ6K && !F::kQ5;
+    // Block minimum, three tiles: the block sums are read from LDS after the products (the same
+    // additions in the same order), because their 16 registers beside the products' spilled
+    // up to 73 others (Q5_K 11008 x 4096, 40 rows: 69.8 -> 35.4 us).
+    constexpr bool kSumsLast = F::kMin && kNT >= 3;
     constexpr int kCopies = 8;           // 1 KB copies per item
     constexpr int kItemB = kCopies * 1024;
     // One array per slot: the compiler then sees that a copy into one does not alias the
@@ -860,7 +865,7 @@ __global__ __launch_bounds__(64 * W * kRH, 2) void gemv_rows_kernel(const uint8_
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const f32x4 rs = *reinterpret_cast<const f32x4*>(my_scale + kq * 4);
         f32x4 bs[4];
-        if constexpr (F::kMin) {
+        if constexpr (F::kMin && !kSumsLast) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) bs[t] = *reinterpret_cast<const f32x4*>(my_sums + t * 16 + kq * 4);
         }
@@ -888,12 +893,23 @@ __global__ __launch_bounds__(64 * W * kRH, 2) void gemv_rows_kernel(const uint8_
                 }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[mg][i][r] = fmaf(gs[r], rs[r], acc[mg][i][r]);
-                if constexpr (F::kMin) {
+                if constexpr (F::kMin && !kSumsLast) {
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) acc[mg][i][r] = fmaf(O.os[i][t], bs[t][r], acc[mg][i][r]);
                 }
+            }
+        }
+        if constexpr (kSumsLast) {
+            fence();
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const f32x4 b = *reinterpret_cast<const f32x4*>(my_sums + t * 16 + kq * 4);
+#pragma unroll
+                for (int i = 0; i < kNT; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[mg][i][r] = fmaf(O.os[i][t], b[r], acc[mg][i][r]);
             }
         }
         // the next item rewrites my_scale after these reads (in-order LDS per wave)
@@ -986,30 +1002,10 @@ bool use_batch_kernel(const Weight& w, int64_t batch) {
     return batch >= kBatchMin && (int64_t)kBatchRows * w.k * 4 <= INT32_MAX;
 }
 
-// The multi-row-group launch of a weight (or pair): T row tiles and W K slices per
-// workgroup.  The waves cut K as a 16-row call's do, so a row has the same bits in either:
-// its own wave count, or eight slices in place of a two-way split over four-wave
-// workgroups (gemv_batch_kernel's halves).  Splits with more waves than that, and K of
-// fewer than 8 groups (one wave), have no such form and stay on 16-row passes (w = 0).  So do
-// weights of more than 768 row tiles: one pass holds at most 3 tiles per workgroup, 16-row
-// passes up to 8, and the activation split is shared by fewer tiles than the saved passes
-// win back (28672 x 8192, 20 / 40 rows: 75 / 109 us against 63 / 98); a pair, at one tile of
-// each weight, from 512 on (11008 x 4096, 20 / 40 rows: 39.7 / 51.4 us against 32.3 / 50.3).
-constexpr int kRowsMax = 4 * kBatchRows;  // rows of one multi-row-group launch
-struct RowsShape {
-    int t = 1, w = 0;
-};
+static_assert(kPassRows == kBatchRows, "a row group is a 16-row call");
 static RowsShape choose_rows_shape(const Weight& w, bool pair) {
     const BatchShape sh = choose_batch_shape(w, kBatchRows, pair);
-    RowsShape r;
-    const int64_t per_cu = (w.n_tiles + kCUs - 1) / kCUs;
-    if (per_cu > (pair ? 2 : 3)) return r;
-    if (sh.split == 1 && sh.w >= 4)
-        r.w = sh.w;
-    else if (sh.split == 2 && sh.w == 4)
-        r.w = 8;
-    r.t = pair ? 1 : (int)per_cu;
-    return r;
+    return rows_shape(w.type, w.n_tiles, w.groups, sh.split, sh.w, pair);
 }
 
 // Four K slices run two row halves of waves (kGroups / 2 row groups each), eight one.
@@ -1017,10 +1013,12 @@ template <int kFmt, int kGroups>
 static hipError_t dispatch_rows(const Weight& w, const Weight* up, const float* x, float* y, int batch,
                                 const RowsShape& sh, hipStream_t s) {
     if (up) return sh.w == 4 ? run_rows<kFmt, 1, 4, 2, 2, kGroups / 2>(w, up->chunks, x, y, batch, s) : hipErrorInvalidValue;
-#define QMM_ROWS_CASE(T_)                                                                             \
-    if (sh.t == T_)                                                                                   \
-        return sh.w == 8 ? run_rows<kFmt, T_, 8, 1, 1, kGroups>(w, nullptr, x, y, batch, s)           \
-                         : run_rows<kFmt, T_, 4, 1, 2, kGroups / 2>(w, nullptr, x, y, batch, s);
+#define QMM_ROWS_CASE(T_)                                                                                          \
+    if (sh.t == T_) {                                                                                              \
+        if (sh.w == 4) return run_rows<kFmt, T_, 4, 1, 2, kGroups / 2>(w, nullptr, x, y, batch, s);                \
+        if constexpr (!(BFmt<kFmt>::kMin && T_ == 3 && kGroups == 4)) /* would spill; rows_shape stays below it */ \
+            return run_rows<kFmt, T_, 8, 1, 1, kGroups>(w, nullptr, x, y, batch, s);                               \
+    }
     QMM_ROWS_CASE(1)
     QMM_ROWS_CASE(2)
     QMM_ROWS_CASE(3)
@@ -1052,20 +1050,14 @@ static hipError_t launch_rows(const Weight& w, const Weight* up, const float* x,
 hipError_t launch_gemv_rows(const Weight& w, const Weight* up, const float* x, float* y, int64_t batch,
                             hipStream_t s) {
     if (use_batch_kernel(w, batch)) {
-        const RowsShape rows = choose_rows_shape(w, up != nullptr);
-        // A pair holds two weights' operands per tile, so one tile per workgroup: that pays
-        // from three row groups on (Q5_K 8192 x 4096, 20 / 40 rows: 36.9 -> 39.8, 58.3 -> 49.9 us).
-        const int64_t least = up ? 2 * kBatchRows : kBatchRows;
-        const bool multi = rows.w != 0 && (int64_t)kRowsMax * w.k * 4 <= INT32_MAX;  // 31-bit x offsets
+        RowsShape rows = choose_rows_shape(w, up != nullptr);
+        if ((int64_t)kRowsMax * w.k * 4 > INT32_MAX) rows.w = 0;  // 31-bit x offsets
         for (int64_t b0 = 0; b0 < batch;) {
-            const int64_t rest = batch - b0;
-            const bool many = multi && rest > least;
-            const int64_t most = many ? kRowsMax : kBatchRows;
-            const int nb = (int)(rest < most ? rest : most);
+            const int nb = next_rows(rows, batch - b0);
             const float* xs = x + b0 * w.k;
             float* ys = y + b0 * w.n;
-            const hipError_t e = many ? launch_rows(w, up, xs, ys, nb, rows, s)
-                                      : launch_gemv_batch(w, up, xs, ys, nb, choose_batch_shape(w, nb, up), s);
+            const hipError_t e = nb > kBatchRows ? launch_rows(w, up, xs, ys, nb, rows, s)
+                                                 : launch_gemv_batch(w, up, xs, ys, nb, choose_batch_shape(w, nb, up), s);
             if (e != hipSuccess) return e;
             b0 += nb;
         }

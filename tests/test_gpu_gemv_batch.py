@@ -360,6 +360,26 @@ def test_many_rows_equal_16_row_calls(qmm, orc, qtype, N, K, B):
     assert_parity(y[rows], orc.linear_f64(qtype, b0, N, K, x[rows]), TOL, f"{qtype} {N}x{K} B={B}")
 
 
+@pytest.mark.parametrize("qtype", [3, 13])
+@pytest.mark.parametrize("N,K,B", [
+    (8200, 1280, 24), (8200, 8192, 40),   # three tiles: four slices, eight slices in two launches
+    (1500, 12288, 20), (1500, 12288, 64)])  # one tile of a two-way split: 16-row passes, one pass
+def test_many_rows_block_minimum(qmm, orc, qtype, N, K, B):
+    """The forms that types with a block minimum run alone: with three tiles the block sums are
+    added after the products, in at most 32 rows where eight slices cut K; long K stays on
+    16-row passes.  A row has the bits of a 16-row call either way."""
+    blocks = (synth.kquant_blocks if qtype == 13 else synth.weight_blocks)(qtype, N, K, seed=0xBD0 + N + K)
+    w = qmm.QuantizedWeight(qtype, blocks, N, K)
+    x = synth.normal(0xBD1 + B, (B, K), 1.0)
+    print(f"many rows, block minimum: type={qtype} N={N} K={K} B={B}", flush=True)
+    y = run_gemv(qmm, w, x)
+    for lo in range(0, B, 16):
+        hi = min(B, lo + 16)
+        assert np.array_equal(y[lo:hi].view(np.uint32), run_gemv(qmm, w, x[lo:hi]).view(np.uint32)), (lo, hi)
+    rows = [0, 15, 16, B - 1]
+    assert_parity(y[rows], orc.linear_f64(qtype, blocks, N, K, x[rows]), TOL, f"{qtype} {N}x{K} B={B}")
+
+
 def test_many_rows_nonfinite_and_ragged(qmm):
     """Rows holding inf / NaN keep to themselves across row groups, and a last K group of
     fewer than 4 blocks reads nothing past a row (x ends in a NaN tail)."""
