@@ -570,81 +570,159 @@ __global__ __launch_bounds__(64 * kNW * kKS, (kGemmWaves<kFmt, kBM, kNW, kWT, kX
     }
     __builtin_amdgcn_s_waitcnt(vmcnt_only(0));  // no copy may land after the stages are reused
 
-    // ---- K parts meet in LDS (the stages are free after this barrier), then store.
-    // Parts 1.. hand their sums over as one 16-byte LDS write per subtile and lane;
-    // part 0 issues all its LDS reads together, adds the parts in order (fixed, so the
-    // bits do not depend on timing) and stores.
+    // ---- K parts meet in LDS (the stages are free after this barrier), then store.  A part
+    // hands its sums of a subtile over as one 16-byte LDS write per lane; they are added in part
+    // order (fixed, so the bits do not depend on timing).  Lane holds D[4 kq + r][li] of each
+    // 16 x 16 subtile.
+    // Four and eight parts: the slice's subtiles are dealt out, subtile q to part q % kKS, so that
+    // the sums, the gate and the stores run on all waves and not on one in kKS (fp32 x, Q8_0
+    // 5632 x 2048 gate and up at 160 rows 54.7 -> 44.9 us; bf16 x, Q8_0 3072 x 2048 at 384 rows
+    // 14.3 -> 13.7; 0.4 - 0.6 us on every size of these shapes).
+    // Two parts: part 0 takes all; dealt out, the 128-row tiles had to spill in the main loop
+    // (split x, Q8_0 11008 x 4096 at 384 rows 94 -> 109 us) and the others gained nothing.
     __syncthreads();
-    auto slot = [&](int h, int i, int j) {
-        const int l = (h - 1) * kMI * kWT + i * kWT + j, arr = l / S::kSlotsPerStage;
-        uint8_t* base = arr == 0 ? lds0 : lds1;
-        return reinterpret_cast<f32x4*>(base) + ((l % S::kSlotsPerStage) * kNW + wn) * 64 + lane;
-    };
+    auto all = [](int, int, int) { return true; };
+    if constexpr (kKS > 2) {
+        // lane indexes of their own: the main loop's would have to live across it
+        const int ln = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), lr = ln & 15, lq = ln >> 4;
+        constexpr int kSub = kMI * kWT, kOwn = kSub / kKS;  // subtiles of the slice, of a part
+        static_assert(kSub % kKS == 0 && (kKS == 4 || kKS == 8), "every K part takes the same number of subtiles");
+        auto slot = [&](int part, int q) {
+            const int owner = q % kKS, l = q * (kKS - 1) + (part < owner ? part : part - 1), arr = l / S::kSlotsPerStage;
+            uint8_t* base = arr == 0 ? lds0 : lds1;
+            return reinterpret_cast<f32x4*>(base) + ((l % S::kSlotsPerStage) * kNW + wn) * 64 + ln;
+        };
+        auto out = [&](int i, int j) { return y + (size_t)(m0 + i * 16 + lq * 4) * n_rows + (tile0 + j) * kTileRows + lr; };
+        auto some = [&](int i, int j, int r) {
+            return m0 + i * 16 + lq * 4 + r < m_rows && (tile0 + j) * kTileRows + lr < n_rows;
+        };
+        auto finish = [&](auto own, auto gated, auto inside) {
+            constexpr int h = decltype(own)::value;
+            // split x: the row scale 2^-e; these and the gate's loads on their way before the first sum
+            int rexp[kX2 ? kMI : 1][4];
+            if constexpr (kX2) {
 #pragma unroll
-    for (int h = 1; h < kKS; ++h)
-        if (kh == h) {
+                for (int i = 0; i < kMI; ++i)
 #pragma unroll
-            for (int i = 0; i < kMI; ++i)
+                    for (int r = 0; r < 4; ++r) rexp[i][r] = -x_exp[min(m0 + i * 16 + lq * 4 + r, m_rows - 1)];
+            }
+            float gate[kOwn][4];
+            if constexpr (gated) {
 #pragma unroll
-                for (int j = 0; j < kWT; ++j) *slot(h, i, j) = acc[i][j];
-        }
-    __syncthreads();
-    if (kh == 0) {
+                for (int o = 0; o < kOwn; ++o) {
+                    const int q = o * kKS + h, i = q / kWT, j = q % kWT;
 #pragma unroll
-        for (int h = 1; h < kKS; ++h) {
-            fence();
-            f32x4 part[kMI][kWT];  // all of a part's reads in flight before the first add
-#pragma unroll
-            for (int i = 0; i < kMI; ++i)
-#pragma unroll
-                for (int j = 0; j < kWT; ++j) part[i][j] = *slot(h, i, j);
-#pragma unroll
-            for (int i = 0; i < kMI; ++i)
-#pragma unroll
-                for (int j = 0; j < kWT; ++j) acc[i][j] += part[i][j];
-        }
-        // split x: the row scale 2^-e of each of the lane's output rows
-        int rexp[kX2 ? kMI : 1][4];
-        if constexpr (kX2) {
-#pragma unroll
-            for (int i = 0; i < kMI; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) rexp[i][r] = -x_exp[min(m0 + i * 16 + kq * 4 + r, m_rows - 1)];
-        }
-        // lane holds D[4 kq + r][li] of each 16 x 16 subtile; a row subtile's gate values
-        // are read together, before its first store
-        auto put = [&](int j, auto gated, auto inside) {
-#pragma unroll
-            for (int i = 0; i < kMI; ++i) {
-                float* yp = y + (size_t)(m0 + i * 16 + kq * 4) * n_rows + (tile0 + j) * kTileRows + li;
-                float gate[4] = {0.f, 0.f, 0.f, 0.f};
-                if constexpr (gated) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (inside(i, j, r)) gate[r] = yp[(size_t)r * n_rows];
+                    for (int r = 0; r < 4; ++r) gate[o][r] = inside(i, j, r) ? out(i, j)[(size_t)r * n_rows] : 0.0f;
                 }
+            }
+#pragma unroll
+            for (int o = 0; o < kOwn; ++o) {
+                const int q = o * kKS + h, i = q / kWT, j = q % kWT;
+                f32x4 sum = h == 0 ? acc[i][j] : *slot(0, q);
+#pragma unroll
+                for (int part = 1; part < kKS; ++part) sum += part == h ? acc[i][j] : *slot(part, q);
+                float* yp = out(i, j);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = acc[i][j][r];
+                    float v = sum[r];
                     if constexpr (kX2) v = __builtin_amdgcn_ldexpf(v, rexp[i][r]);
-                    if constexpr (gated) v = gate[r] / (1.0f + expf(-gate[r])) * v;
+                    if constexpr (gated) v = gate[o][r] / (1.0f + expf(-gate[o][r])) * v;
                     if (inside(i, j, r)) yp[(size_t)r * n_rows] = v;
                 }
             }
         };
-        auto all = [](int, int, int) { return true; };
-        auto some = [&](int i, int j, int r) {
-            return m0 + i * 16 + kq * 4 + r < m_rows && (tile0 + j) * kTileRows + li < n_rows;
+#pragma unroll
+        for (int h = 0; h < kKS; ++h)
+            if (kh == h) {
+#pragma unroll
+                for (int q = 0; q < kSub; ++q)
+                    if (q % kKS != h) *slot(h, q) = acc[q / kWT][q % kWT];
+            }
+        __syncthreads();
+        auto part = [&](auto own) {
+            if (kh != decltype(own)::value) return;
+            if (gate_in_y)
+                finish(own, std::true_type{}, some);
+            else if (m0 + kBM <= m_rows && (tile0 + kWT) * kTileRows <= n_rows)  // whole tile inside y
+                finish(own, std::false_type{}, all);
+            else
+                finish(own, std::false_type{}, some);
         };
-        if (m0 + kBM <= m_rows && (tile0 + kWT) * kTileRows <= n_rows && !gate_in_y) {  // whole tile inside y
+        part(std::integral_constant<int, 0>{});
+        part(std::integral_constant<int, 1>{});
+        part(std::integral_constant<int, 2>{});
+        part(std::integral_constant<int, 3>{});
+        if constexpr (kKS == 8) {
+            part(std::integral_constant<int, 4>{});
+            part(std::integral_constant<int, 5>{});
+            part(std::integral_constant<int, 6>{});
+            part(std::integral_constant<int, 7>{});
+        }
+    } else {
+        auto slot = [&](int i, int j) {
+            const int l = i * kWT + j, arr = l / S::kSlotsPerStage;
+            uint8_t* base = arr == 0 ? lds0 : lds1;
+            return reinterpret_cast<f32x4*>(base) + ((l % S::kSlotsPerStage) * kNW + wn) * 64 + lane;
+        };
+        if (kh == 1) {
 #pragma unroll
-            for (int j = 0; j < kWT; ++j) put(j, std::false_type{}, all);
-        } else if (!gate_in_y) {
+            for (int i = 0; i < kMI; ++i)
 #pragma unroll
-            for (int j = 0; j < kWT; ++j) put(j, std::false_type{}, some);
-        } else {
+                for (int j = 0; j < kWT; ++j) *slot(i, j) = acc[i][j];
+        }
+        __syncthreads();
+        if (kh == 0) {
+            fence();
+            f32x4 part[kMI][kWT];  // all reads in flight before the first add
 #pragma unroll
-            for (int j = 0; j < kWT; ++j) put(j, std::true_type{}, some);
+            for (int i = 0; i < kMI; ++i)
+#pragma unroll
+                for (int j = 0; j < kWT; ++j) part[i][j] = *slot(i, j);
+#pragma unroll
+            for (int i = 0; i < kMI; ++i)
+#pragma unroll
+                for (int j = 0; j < kWT; ++j) acc[i][j] += part[i][j];
+            // split x: the row scale 2^-e of each of the lane's output rows
+            int rexp[kX2 ? kMI : 1][4];
+            if constexpr (kX2) {
+#pragma unroll
+                for (int i = 0; i < kMI; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) rexp[i][r] = -x_exp[min(m0 + i * 16 + kq * 4 + r, m_rows - 1)];
+            }
+            // a row subtile's gate values are read together, before its first store
+            auto put = [&](int j, auto gated, auto inside) {
+#pragma unroll
+                for (int i = 0; i < kMI; ++i) {
+                    float* yp = y + (size_t)(m0 + i * 16 + kq * 4) * n_rows + (tile0 + j) * kTileRows + li;
+                    float gate[4] = {0.f, 0.f, 0.f, 0.f};
+                    if constexpr (gated) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (inside(i, j, r)) gate[r] = yp[(size_t)r * n_rows];
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        float v = acc[i][j][r];
+                        if constexpr (kX2) v = __builtin_amdgcn_ldexpf(v, rexp[i][r]);
+                        if constexpr (gated) v = gate[r] / (1.0f + expf(-gate[r])) * v;
+                        if (inside(i, j, r)) yp[(size_t)r * n_rows] = v;
+                    }
+                }
+            };
+            auto some = [&](int i, int j, int r) {
+                return m0 + i * 16 + kq * 4 + r < m_rows && (tile0 + j) * kTileRows + li < n_rows;
+            };
+            if (m0 + kBM <= m_rows && (tile0 + kWT) * kTileRows <= n_rows && !gate_in_y) {
+#pragma unroll
+                for (int j = 0; j < kWT; ++j) put(j, std::false_type{}, all);
+            } else if (!gate_in_y) {
+#pragma unroll
+                for (int j = 0; j < kWT; ++j) put(j, std::false_type{}, some);
+            } else {
+#pragma unroll
+                for (int j = 0; j < kWT; ++j) put(j, std::true_type{}, some);
+            }
         }
     }
 }

@@ -271,6 +271,38 @@ def test_gemm_every_launch_shape(qmm, orc, qtype, split_x):
     assert sorted(seen) == expect, seen
 
 
+@pytest.mark.parametrize("qtype", [Q4_0, Q8_0, Q6_K])
+@pytest.mark.parametrize("N,M,K", [(100, 5, 512), (8251, 65, 1024), (8251, 5, 512), (8251, 65, 256), (12347, 200, 256)])
+def test_gate_epilogue_of_every_k_split(qmm, qtype, N, M, K):
+    """silu(gate) * up in the up GEMM's epilogue (fp32 and bf16 x) on shapes of two, four and
+    eight K parts: from the two products' own bits, within the rounding of exp and the
+    quotient (1e-6)."""
+    L = _native.lib()
+    g, u = (qmm.QuantizedWeight(qtype, blocks_for(qtype, N, K, seed=0xFB0 + i + N), N, K) for i in (0, 1))
+    x = synth.normal(0xFB2 + M, (M, K), 1.0)
+    xb = synth.to_bf16_bits(x)
+    dx, dxb, dh = qmm.DeviceBuffer.from_numpy(x), qmm.DeviceBuffer.from_numpy(xb), qmm.DeviceBuffer(M * N * 4)
+    work = qmm.gemm_f32_workspace(M, K)
+    for split in (1, 0):
+        shape = L.openmini_qmm_gemm_launch_shape(u.handle, M, split)
+        print(f"gate epilogue type={qtype} N={N} M={M} K={K} split={split} shape={shape}", flush=True)
+        dh.fill(0xFF)
+        if split:
+            _native.check(L.openmini_qmm_ffn_gate_up_f32(g.handle, u.handle, dx.ptr, dh.ptr, M, work.ptr, work.nbytes, None))
+            yg, yu = run_gemm_f32(qmm, g, x), run_gemm_f32(qmm, u, x)
+        else:
+            _native.check(L.openmini_qmm_ffn_gate_up_bf16(g.handle, u.handle, dxb.ptr, dh.ptr, M, None))
+            ys = []
+            for w in (g, u):
+                dy = qmm.DeviceBuffer(M * N * 4)
+                w.gemm_bf16(dxb, dy, M)
+                ys.append(dy.download(np.float32, (M, N)))
+            yg, yu = ys
+        h = dh.download(np.float32, (M, N))
+        ref = yg.astype(np.float64) / (1.0 + np.exp(-yg.astype(np.float64))) * yu
+        assert np.all(np.abs(h - ref) <= 1e-6 * np.abs(ref) + 1e-30)
+
+
 @pytest.mark.parametrize("qtype,N,K,M", [
     (Q4_0, 33, 32, 1), (Q8_0, 31, 96, 17),         # fewer K groups than K parts, a ragged last group
     (Q4_0, 200, 1120, 63), (Q8_0, 65, 1120, 129),  # a part without a last group; a row past a tile
