@@ -222,10 +222,11 @@ int openmini_qmm_gemm_bf16(const openmini_qweight_t* weight, const uint16_t* d_x
 size_t openmini_qmm_gemm_f32_workspace_bytes(int64_t m, int64_t k_cols);
 
 /* Diagnostic, no counterpart in the reference: the launch shape the prefill GEMM picks
- * for m rows on this weight (bf16 activations, or split fp32 ones when split_x != 0):
- * rows per workgroup x columns per wave, 0 = 128 x 48, 1 = 128 x 32, 2 = 64 x 48, 3 =
- * 64 x 32 (eight waves per workgroup, splitting its columns and K), chosen from the problem size alone, so a row's bits depend only on m and
- * the weight.  A negative status on error. */
+ * for m rows on this weight (bf16 activations, or split fp32 ones when split_x != 0), as
+ * rows x columns of a workgroup: 0 = 128 x 192, 1 = 128 x 128, 2 = 64 x 96, 3 = 64 x 128,
+ * 4 = 64 x 64, 5 = 64 x 32 (eight waves each, splitting its columns and K), 6 = 64 x 64 and
+ * 7 = 128 x 96 in four waves.  Chosen from the problem size alone, so a row's bits depend only on m and the
+ * weight.  A negative status on error. */
 int openmini_qmm_gemm_launch_shape(const openmini_qweight_t* weight, int64_t m, int split_x);
 
 /* Routing query, no counterpart in the reference: the fewest activation rows from which

@@ -17,11 +17,11 @@
 // MFMA's 32, so q * scale (an exact integer of at most 13 bits) enters as bf16
 // hi + lo (two chained MFMAs, both exact), and the row's d is the block factor.
 //
-// Tiling: a workgroup of eight waves computes a kBM x (16 kWT kNW) tile of y with kNW
-// column slices x kKS K parts of waves (choose_shape picks one of six shapes, 128 x 192 to
-// 64 x 32, by problem size).  A wave owns kBM rows x 16 kWT columns (kBM/16 x kWT MFMA
-// subtiles of fp32 accumulators) over one K part, and the parts are added through
-// LDS at the end (fixed order).  A K step is two blocks (64 elements):
+// Tiling: a workgroup of eight waves (four in two shapes) computes a kBM x (16 kWT kNW) tile
+// of y with kNW column slices x kKS K parts of waves (choose_gemm_shape picks one of eight
+// shapes, 128 x 192 to 64 x 32, by problem size).  A wave owns kBM rows x 16 kWT columns
+// (kBM/16 x kWT MFMA subtiles of fp32 accumulators) over one K part, and the parts are added
+// through LDS at the end (fixed order).  A K step is two blocks (64 elements):
 //   * x: each K part's kBM x 64 bf16 slab is copied HBM -> LDS by buffer loads with
 //     an LDS destination (no registers) two steps ahead, rows XOR-swizzled in 16-byte
 //     segments so the A-fragment reads are bank-conflict free; the fragments of a half
@@ -40,6 +40,7 @@
 // hid those waits, gained most: Q8_0 4096 x 11008 at 100 fp32 rows 92 -> 40 us (with the
 // 64 x 32 shape, which fills the chip there).
 #include "qmm_device.hpp"
+#include "qmm_gemm_shape.hpp"
 
 #include <type_traits>
 
@@ -738,52 +739,6 @@ hipError_t launch_shape(const Weight& w, const uint16_t* x, const int* x_exp, fl
     return hipGetLastError();
 }
 
-// Launch shapes: eight waves each, as column slices x K parts.
-//   0: 128 x 192 tiles, 4 x 2 waves, 3 weight tiles per wave   3:  64 x 128, 4 x 2 waves, 2 tiles
-//   1: 128 x 128, 4 x 2 waves, 2 tiles                        4:  64 x  64, 2 x 4 waves, 2 tiles
-//   2:  64 x  96, 2 x 4 waves, 3 tiles                        5:  64 x  32, 1 x 8 waves, 2 tiles
-constexpr int kShapes = 6;
-constexpr int kShapeRows[kShapes] = {128, 128, 64, 64, 64, 64};
-constexpr int kShapeTiles[kShapes] = {12, 8, 6, 8, 4, 2};  // weight tiles (16 columns) per workgroup
-// Launch shape by problem size.  Few and large workgroups leave CUs idle or a last round
-// part-filled; small ones cost more per flop (each B fragment serves fewer MFMAs, each A
-// fragment fewer tiles).  The model: workgroups run in rounds of 256 CUs x one (or two,
-// where the kernel's registers let two share a CU: 64 x 128 and 64 x 64); a round costs
-// the shape's time per K element, measured on MI355X over 15 weight shapes x 100..1024
-// rows (Q4_0 / Q8_0 / Q4_K, and Q6_K, whose blocks run two to four MFMAs, on its own):
-// kOne for one workgroup on a CU, kTwo for two, plus kExtra for a workgroup's start and
-// K-part sums where that decides (64 x 96 at short K).  It picks the fastest shape or one
-// within 3% of it at every size measured; e.g. fp32 x, 100 rows of Q8_0 4096 x 11008: 64 x
-// 32 40.3 us, 64 x 64 63.1, 64 x 96 78.8, 64 x 128 97.7, 128 x 128 155, 128 x 192 216; bf16
-// x, 1024 rows of Q4_0 28672 x 8192: 128 x 192 566 us, 128 x 128 585, 64 x 128 622, 64 x 64
-// 696.  Fixed per shape, so a row's bits depend only on m and the weight.  A shape with
-// per_cu < 0 is not built for the instance: Q6_K on bf16 x has no 128 x 192 tiles (its
-// super-block sums would not fit the registers).
-int choose_shape(const Weight& w, int64_t m, const int (&per_cu)[kShapes], bool split_x) {
-    static const double kOne[4][kShapes] = {{13.8, 9.8, 4.8, 5.9, 3.4, 2.0},      // bf16 x
-                                            {0.0, 14.3, 8.2, 10.3, 5.7, 3.4},     // bf16 x, Q6_K
-                                            {21.8, 15.6, 7.0, 8.25, 5.2, 3.0},    // split x
-                                            {34.0, 23.2, 11.3, 14.4, 7.8, 4.9}};  // split x, Q6_K
-    static const double kTwo[2][kShapes] = {{0, 0, 0, 10.8, 5.9, 0}, {0, 0, 0, 15.9, 8.8, 0}};
-    static const double kExtra[4] = {500.0, 500.0, 1000.0, 1700.0};  // ns, shape 2
-    constexpr int64_t kCus = 256;
-    const int row = (split_x ? 2 : 0) + (w.type == OPENMINI_QMM_Q6_K ? 1 : 0);
-    int best = -1;
-    double best_cost = 0.0;
-    for (int i = 0; i < kShapes; ++i) {
-        if (per_cu[i] < 0) continue;
-        const int64_t wgs = (w.n_tiles + kShapeTiles[i] - 1) / kShapeTiles[i] * ((m + kShapeRows[i] - 1) / kShapeRows[i]);
-        const double one = kOne[row][i];
-        const bool pairs = per_cu[i] >= 2 && kTwo[split_x][i] > 0.0;
-        const double full = pairs ? kTwo[split_x][i] : one;
-        const int64_t slots = pairs ? 2 * kCus : kCus, left = wgs % slots;
-        double cost = ((double)(wgs / slots) * full + (left > kCus ? full : left ? one : 0.0)) * (double)w.k;
-        if (i == 2) cost += kExtra[row];
-        if (best < 0 || cost < best_cost) best = i, best_cost = cost;
-    }
-    return best;
-}
-
 // Workgroups of `kernel` (at `threads` per workgroup) one CU holds at once.
 int blocks_per_cu(const void* kernel, int threads) {
     int n = 0;
@@ -791,7 +746,8 @@ int blocks_per_cu(const void* kernel, int threads) {
     return n;
 }
 
-// Shape 0 is built for every instance but Q6_K on bf16 x.
+// Shapes 0 and 7 (128 rows x 3 weight tiles per wave) are built for every instance but Q6_K on
+// bf16 x, whose super-block sums would not fit the registers.
 template <int kFmt, bool kX2>
 constexpr bool kWideTiles = kFmt != OPENMINI_QMM_Q6_K || kX2;
 
@@ -804,19 +760,27 @@ const int (&shape_occupancy())[kShapes] {
         else
             return -1;
     };
+    auto narrow = [] {
+        if constexpr (kWideTiles<kFmt, kX2>)
+            return blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 2, 2, 3, kX2>, 256);
+        else
+            return -1;
+    };
     static const int per_cu[kShapes] = {wide(),
                                         blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 4, 2, 2, kX2>, 512),
                                         blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 4, 3, kX2>, 512),
                                         blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 4, 2, 2, kX2>, 512),
                                         blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 4, 2, kX2>, 512),
-                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 1, 8, 2, kX2>, 512)};
+                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 1, 8, 2, kX2>, 512),
+                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 2, 2, kX2>, 256),
+                                        narrow()};
     return per_cu;
 }
 
 template <int kFmt, bool kX2>
 hipError_t launch_kind(const Weight& w, const uint16_t* x, const int* x_exp, float* y, int64_t m, bool gate,
                        hipStream_t s) {
-    switch (choose_shape(w, m, shape_occupancy<kFmt, kX2>(), kX2)) {
+    switch (choose_gemm_shape(w.type, w.n_tiles, w.k, m, shape_occupancy<kFmt, kX2>(), kX2)) {
     case 0:
         if constexpr (kWideTiles<kFmt, kX2>) return launch_shape<kFmt, 128, 4, 2, 3, kX2>(w, x, x_exp, y, m, gate, s);
         return hipErrorInvalidValue;
@@ -824,7 +788,12 @@ hipError_t launch_kind(const Weight& w, const uint16_t* x, const int* x_exp, flo
     case 2: return launch_shape<kFmt, 64, 2, 4, 3, kX2>(w, x, x_exp, y, m, gate, s);
     case 3: return launch_shape<kFmt, 64, 4, 2, 2, kX2>(w, x, x_exp, y, m, gate, s);
     case 4: return launch_shape<kFmt, 64, 2, 4, 2, kX2>(w, x, x_exp, y, m, gate, s);
-    default: return launch_shape<kFmt, 64, 1, 8, 2, kX2>(w, x, x_exp, y, m, gate, s);
+    case 5: return launch_shape<kFmt, 64, 1, 8, 2, kX2>(w, x, x_exp, y, m, gate, s);
+    case 6: return launch_shape<kFmt, 64, 2, 2, 2, kX2>(w, x, x_exp, y, m, gate, s);
+    case 7:
+        if constexpr (kWideTiles<kFmt, kX2>) return launch_shape<kFmt, 128, 2, 2, 3, kX2>(w, x, x_exp, y, m, gate, s);
+        return hipErrorInvalidValue;
+    default: return hipErrorInvalidValue;
     }
 }
 
@@ -1052,9 +1021,8 @@ hipError_t launch_gemm_bf16(const Weight& w, const uint16_t* x, float* y, int64_
 int gemm_shape(const Weight& w, int64_t m, bool split_x) {
     auto pick = [&](auto fmt) {
         constexpr int kFmt = decltype(fmt)::value;
-        const int i = split_x ? choose_shape(w, m, shape_occupancy<kFmt, true>(), true)
-                              : choose_shape(w, m, shape_occupancy<kFmt, false>(), false);
-        return i > 3 ? 3 : i;  // by rows per workgroup and weight tiles per wave
+        return split_x ? choose_gemm_shape(kFmt, w.n_tiles, w.k, m, shape_occupancy<kFmt, true>(), true)
+                       : choose_gemm_shape(kFmt, w.n_tiles, w.k, m, shape_occupancy<kFmt, false>(), false);
     };
     switch (w.type) {
     case OPENMINI_QMM_Q4_0: return pick(std::integral_constant<int, OPENMINI_QMM_Q4_0>{});

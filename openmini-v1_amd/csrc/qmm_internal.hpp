@@ -291,7 +291,7 @@ hipError_t launch_gemm_bf16(const Weight& w, const uint16_t* x, float* y, int64_
 // hi / lo parts plus a per-row exponent into `work` (gemm_f32_workspace_bytes(m, k)
 // bytes, 256-byte aligned), launch_gemm_split runs the GEMM on them.
 size_t gemm_f32_workspace_bytes(int64_t m, int64_t k);
-// The prefill GEMM's launch shape (0..3 by rows and columns per wave, qmm_gemm.hip choose_shape) for m rows of bf16
+// The prefill GEMM's launch shape (index into kShapeRows, qmm_gemm_shape.hpp) for m rows of bf16
 // (split_x false) or split fp32 (true) activations; -1 for a type it does not take.
 int gemm_shape(const Weight& w, int64_t m, bool split_x);
 // For weights of w's type and K.

@@ -233,25 +233,42 @@ def test_gemm_f32_workspace_checks(qmm):
     assert L.openmini_qmm_gemm_f32_workspace_bytes(0, K) == 0
 
 
-@pytest.mark.parametrize("split_x", [False, True])
-@pytest.mark.parametrize("qtype", [Q4_0, Q8_0, Q4_K, Q6_K])
+# (type, split fp32 x): launch shape -> the smallest size (N, M, K) found that picks it, last
+# row tiles ragged.  Shapes that are not listed for a type are picked only at larger sizes, or
+# not built (0 and 7 for Q6_K on bf16 x, whose super-block sums would not fit the registers).
+SHAPE_SIZES = {
+    (Q4_0, False): {1: (12347, 200, 2048), 2: (8251, 65, 1024), 3: (11323, 257, 2048), 4: (8251, 5, 256),
+                    5: (27, 5, 256), 6: (8251, 65, 256), 7: (9275, 513, 512)},
+    (Q8_0, False): {0: (9275, 513, 2048), 1: (12347, 200, 2048), 2: (8251, 65, 1024), 3: (12347, 200, 256),
+                    4: (8251, 5, 512), 5: (27, 5, 256), 6: (8251, 5, 256), 7: (9275, 513, 1024)},
+    (Q4_K, False): {1: (12347, 200, 2048), 2: (8251, 65, 1024), 3: (11323, 257, 2048), 4: (8251, 5, 256),
+                    5: (27, 5, 256), 6: (8251, 65, 256), 7: (9275, 513, 512)},
+    (Q6_K, False): {1: (11323, 129, 512), 2: (8251, 65, 1024), 4: (8251, 5, 512), 5: (27, 5, 256),
+                    6: (8251, 5, 256)},
+    (Q4_0, True): {0: (9275, 513, 1024), 2: (8251, 65, 1024), 3: (12347, 200, 256), 4: (8251, 5, 256),
+                   5: (27, 5, 256), 6: (11323, 129, 256), 7: (13371, 600, 4096)},
+    (Q8_0, True): {0: (13371, 257, 1024), 2: (8251, 65, 2048), 3: (12347, 200, 256), 4: (8251, 5, 256),
+                   5: (27, 5, 256), 6: (11323, 129, 256), 7: (13371, 600, 2048)},
+    (Q4_K, True): {0: (9275, 513, 1024), 2: (8251, 65, 1024), 3: (12347, 200, 256), 4: (8251, 5, 256),
+                   5: (27, 5, 256), 6: (11323, 129, 256), 7: (13371, 600, 4096)},
+    (Q6_K, True): {0: (13371, 257, 1024), 1: (12347, 200, 256), 2: (8251, 65, 512), 3: (12347, 65, 4096),
+                   4: (8251, 5, 256), 5: (27, 5, 256), 6: (8251, 65, 256), 7: (9275, 513, 256)},
+}
+
+
+@pytest.mark.parametrize("qtype,split_x", sorted(SHAPE_SIZES))
 def test_gemm_every_launch_shape(qmm, orc, qtype, split_x):
-    """The prefill GEMM picks one of four launch shapes (128 or 64 rows x 3 or 2 weight
-    tiles per wave) from the problem size.  Over these sizes every shape must be picked
-    at least once, for every weight type, with bf16 and with split fp32 activations,
-    and every call meets the oracle (sampled rows, y NaN-filled).  Q6_K on bf16
-    activations has no 128 x 96 shape (its per-super-block sums would not fit the
-    registers), and split activations no 64 x 96 shape (64 x 64 runs faster or within
-    0.6% there)."""
+    """The prefill GEMM picks one of eight launch shapes from the problem size (128 x 192 to
+    64 x 32 per workgroup, eight or four waves).  Each size picks its shape, and every call
+    meets the oracle: sampled rows, y NaN-filled, ragged last row tiles.  The products are
+    exact, so the outputs differ from fp64 by fp32 sums: 1e-5 of the largest is above 20 times
+    that rounding."""
     L = _native.lib()
-    K = 512
-    seen = {}
-    for N, M in ((100, 5), (4096, 512), (8192, 1024), (11008, 512), (11008, 128)):
+    for shape, (N, M, K) in sorted(SHAPE_SIZES[qtype, split_x].items()):
         blocks = blocks_for(qtype, N, K, seed=0xF70 + N + M)
         w = qmm.QuantizedWeight(qtype, blocks, N, K)
-        shape = L.openmini_qmm_gemm_launch_shape(w.handle, M, int(split_x))
-        assert 0 <= shape <= 3, shape
-        print(f"gemm shape {shape}: type={qtype} split_x={split_x} N={N} M={M}", flush=True)
+        assert L.openmini_qmm_gemm_launch_shape(w.handle, M, int(split_x)) == shape, (shape, N, M, K)
+        print(f"gemm shape {shape}: type={qtype} split_x={split_x} N={N} M={M} K={K}", flush=True)
         x = synth.normal(0xF71 + M, (M, K), 1.0)
         rows = np.unique(np.concatenate([[0, M - 1], np.random.default_rng(N).integers(0, M, 6)]))
         if split_x:
@@ -265,10 +282,7 @@ def test_gemm_every_launch_shape(qmm, orc, qtype, split_x):
             y = dy.download(np.float32, (M, N))
             ref = orc.linear_bf16x_f64(qtype, blocks, N, K, xb[rows])
         assert np.all(np.isfinite(y)), "unwritten (NaN) outputs"
-        assert_parity(y[rows], ref, TOL, f"shape {shape} N={N} M={M}")
-        seen.setdefault(shape, (N, M))
-    expect = [0, 1, 3] if split_x else [1, 2, 3] if qtype == 14 else [0, 1, 2, 3]
-    assert sorted(seen) == expect, seen
+        assert np.max(np.abs(y[rows] - ref)) <= 1e-5 * np.max(np.abs(ref)), (shape, N, M, K)
 
 
 @pytest.mark.parametrize("qtype", [Q4_0, Q8_0, Q6_K])
@@ -310,8 +324,8 @@ def test_gate_epilogue_of_every_k_split(qmm, qtype, N, M, K):
     (Q4_0, 4090, 96, 200), (Q8_0, 4100, 160, 130), (Q6_K, 4100, 256, 200),
     (Q8_0, 8200, 96, 1000), (Q4_K, 11000, 256, 500), (Q6_K, 11000, 256, 400)])
 def test_gemm_tile_edges(qmm, orc, qtype, N, K, M):
-    """Every launch shape at the edges of its tiles, on bf16 and fp32 activations: rows and
-    columns past whole tiles, K parts of zero, one and unequal group counts.  The products
+    """Edges of the tiles, on bf16 and fp32 activations (the shapes one by one:
+    test_gemm_every_launch_shape): rows and columns past whole tiles, K parts of zero, one and unequal group counts.  The products
     are exact, so the outputs differ from fp64 by fp32 sums of at most K / 32 block sums
     of 32 terms: 1e-5 of the largest output is above 20 times that rounding."""
     blocks = blocks_for(qtype, N, K, seed=0xFA0 + N + K + M)

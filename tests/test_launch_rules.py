@@ -1,5 +1,5 @@
-"""The launch rules that are plain C++ (csrc/qmm_rows_shape.hpp), asked on the host: at sizes
-where both ways were measured on MI355X they take the faster one."""
+"""The launch rules that are plain C++ (csrc/qmm_rows_shape.hpp, qmm_gemm_shape.hpp), asked on the
+host: at sizes where the ways were measured on MI355X they take the fastest or one within 3%."""
 import os
 import shutil
 import subprocess
@@ -82,3 +82,61 @@ int main() {
 
 def test_rows_of_a_pass(tmp_path):
     run_program(tmp_path, "rows", ROWS)
+
+
+GEMM = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "qmm_gemm_shape.hpp"
+using namespace qmm;
+
+enum { Q4_0 = 2, Q8_0 = 7, Q4_K = 12, Q6_K = 14 };
+
+// workgroups per CU: what the kernels' registers and LDS allow on gfx950
+static const int kPerCu[6][kShapes] = {{1, 1, 1, 2, 2, 1, 4, 2}, {1, 1, 1, 2, 1, 1, 3, 2}, {-1, 1, 1, 1, 1, 1, 2, -1},
+                                       {1, 1, 1, 2, 2, 1, 4, 2}, {1, 1, 1, 2, 2, 1, 4, 2}, {1, 1, 1, 1, 1, 1, 3, 2}};
+static int pick(int type, int n, int k, int m, bool split) {
+    return choose_gemm_shape(type, (n + 15) / 16, k, m, kPerCu[(split ? 3 : 0) + (type == Q8_0 ? 1 : type == Q6_K ? 2 : 0)], split);
+}
+
+int main() {
+    // measured with every shape forced: those within 3% of the fastest
+    struct { int type, n, k, m; bool split; unsigned good; } cases[] = {
+        {Q8_0, 11008, 2048, 384, true, 1u << 0 | 1u << 7},  // 53 us; 64 x 96 64
+        {Q8_0, 7168, 4096, 600, true, 1u << 0}, {Q8_0, 14336, 4096, 300, true, 1u << 0},
+        {Q8_0, 13824, 4096, 100, true, 1u << 4},
+        {Q8_0, 13824, 4096, 100, false, 1u << 6}, {Q8_0, 11008, 4096, 768, false, 1u << 6 | 1u << 7},
+        {Q8_0, 13824, 4096, 1536, false, 1u << 7}, {Q8_0, 11008, 4096, 512, false, 1u << 0},
+        {Q8_0, 4096, 11008, 100, true, 1u << 5}, {Q4_0, 4096, 4096, 128, false, 1u << 5},
+        {Q6_K, 11008, 2048, 448, false, 1u << 6}};
+    for (const auto& c : cases) {
+        const int got = pick(c.type, c.n, c.k, c.m, c.split);
+        if (got < 0 || !(c.good >> got & 1)) {
+            std::printf("type %d %d x %d, %d rows, split %d: shape %d\n", c.type, c.n, c.k, c.m, c.split, got);
+            return 1;
+        }
+    }
+    // always one that is built, whatever a CU holds of it
+    for (int type : {Q4_0, Q8_0, Q4_K, Q6_K})
+        for (int split = 0; split < 2; ++split)
+            for (int tiles : {1, 2, 100, 688, 2000, 40000})
+                for (int k : {32, 4096, 65536})
+                    for (int m : {1, 64, 65, 300, 4096, 300000})
+                        for (int cu : {0, 1, 2, 8}) {
+                            int per_cu[kShapes];
+                            for (int i = 0; i < kShapes; ++i)
+                                per_cu[i] = !split && type == Q6_K && (i == 0 || i == 7) ? -1 : cu;
+                            const int got = choose_gemm_shape(type, tiles, k, m, per_cu, split);
+                            if (got < 0 || got >= kShapes || per_cu[got] < 0) {
+                                std::printf("type %d tiles %d k %d m %d: shape %d\n", type, tiles, k, m, got);
+                                return 1;
+                            }
+                        }
+    std::printf("ok\n");
+    return 0;
+}
+"""
+
+
+def test_gemm_shape(tmp_path):
+    run_program(tmp_path, "gemm", GEMM)
