@@ -29,6 +29,9 @@ constexpr int kShapeTiles[kShapes] = {12, 8, 6, 8, 4, 2, 4, 6};  // weight tiles
 // CU, are there for the sizes between two rounds of the large tiles: bf16 x, Q8_0 11008 x 4096
 // at 768 rows 122 us without them, 114 in shape 6, 110 in shape 7; 13824 x 4096 at 100 rows
 // 33.1 -> 30.1 in shape 6, at 1536 rows 244 -> 228 in shape 7.
+// (Long runs.  In the first milliseconds after idle the card is slower and small tiles lose
+// more: where Q6_K on bf16 x tied in long runs, 11008 x 4096 at 512 rows 121 us in shapes 1 and
+// 6 but 141 and 154 after idle, shape 6's row is priced 1.5% up.)
 struct ShapeCost {
     double start = 0.0;                 // us of a round
     double per_k[4] = {0., 0., 0., 0.}; // us of a round per 1000 K elements, 1 .. 4 workgroups on a CU
@@ -46,7 +49,7 @@ inline int choose_gemm_shape(int type, int64_t n_tiles, int64_t k, int64_t m, co
          {1.7, {3.46}}, {1.8, {1.92}}, {1.3, {4.39, 6.35, 8.66}}, {4.6, {10.1, 14.6}}},
         // bf16 x: Q6_K (no 128 x 192)
         {{}, {4.1, {13.6}}, {3.1, {7.44}}, {2.2, {9.85}},
-         {2.0, {5.19}}, {2.1, {2.61}}, {1.6, {6.52, 9.30}}, {}},
+         {2.0, {5.19}}, {2.1, {2.61}}, {1.6, {6.60, 9.45}}, {}},
         // split x: Q4_0, Q4_K
         {{5.5, {18.9}}, {4.3, {13.7}}, {2.4, {6.25}}, {1.8, {8.37, 13.9}},
          {0.7, {5.34, 8.31}}, {1.3, {2.99}}, {1.3, {7.07, 8.87, 12.4, 16.0}}, {4.7, {13.8, 20.9}}},
