@@ -183,10 +183,10 @@ int openmini_qmm_weight_info(const openmini_qweight_t* weight,
 
 /* Decode GEMV: y[batch, N] = x[batch, K] . W^T, fp32 activations, fp32 output.
  * Any batch >= 1.  Up to 3 rows: the single-row-tuned kernel; 4 or more: the
- * batched kernels, one pass over W per 16 rows (17 to 64 rows: one pass for all on
- * weights of at most 12288 rows), in which a row's result does not depend on the
- * other rows of the call nor on the batch size (bitwise).  Every
- * weight type.
+ * batched kernels, one pass over W per 16 rows (on weights of at most 12288 rows mostly
+ * one for 17 to 64 rows, by type, shape and rows where that is faster), in which a row's
+ * result does not depend on the other rows of the call nor on the batch size (bitwise).
+ * Every weight type.
  * A weight of at most 8192 rows and K >= 4000 splits K of a batched call over two or
  * four workgroups per row tile; their partial sums and arrival counters live in a
  * mutable workspace after the weight's chunks (counted in device_bytes: 128 or 256 B
@@ -231,11 +231,12 @@ int openmini_qmm_gemm_launch_shape(const openmini_qweight_t* weight, int64_t m, 
 
 /* Routing query, no counterpart in the reference: the fewest activation rows from which
  * openmini_qmm_linear_host (and _noalloc) run the fp32 prefill GEMM on this weight
- * rather than the decode GEMVs: the first m in [64, 128) where the GEMM's estimated
- * time (about 10 ns per K element while its grid fits one round) beats the GEMVs' (one
- * pass per 16 rows, about 6.5 us plus the weight bytes at 3-5 TB/s), else 128; 0 for
- * Q4_1 / Q5_K, which have no prefill GEMM.  Depends on the weight's type and shape
- * only.  Engines that call the GEMM and GEMV entry points themselves use it to make
+ * rather than the decode GEMVs: the first m in [64, 128) where an estimate of the GEMM's
+ * time (10 ns per K element while its grid fits one round) is below one of the GEMVs'
+ * (6.5 us plus the weight bytes at 3-5 TB/s per 16 rows), else 128; 0 for Q4_1 / Q5_K,
+ * which have no prefill GEMM.  Depends on the weight's type and shape only.  The estimates
+ * are older than the kernels: from 65 rows on the GEMM is the faster one on nearly every
+ * weight, most on few rows and long K (Q4_0 1024 x 8192, 96 rows: 32 us against 55).  Engines that call the GEMM and GEMV entry points themselves use it to make
  * the same choice.  A negative status on error. */
 int64_t openmini_qmm_gemm_min_rows(const openmini_qweight_t* weight);
 int openmini_qmm_gemm_f32(const openmini_qweight_t* weight, const float* d_x, float* d_y, int64_t m,
@@ -246,17 +247,17 @@ int openmini_qmm_gemm_f32(const openmini_qweight_t* weight, const float* d_x, fl
 /* Weights that share the input: d_ys[i][batch, N_i] = x[batch, K] . W_i^T for
  * i < count (1..4), all of one type and one K; one launch for up to 3 batch rows and,
  * for weights that together fill the chip once, for 4 to 16, else one batched pass per
- * weight (results identical to openmini_qmm_gemv of each weight).  Replaces the three linear_gemm calls of prepare_qkv
- * (model.rs:1392-1394: q, k, v of one normalised hidden state).  d_x must be
- * 16-byte aligned. */
+ * weight (results identical to openmini_qmm_gemv of each weight).  Replaces the three
+ * linear_gemm calls of prepare_qkv (model.rs:1392-1394: q, k, v of one normalised hidden
+ * state).  d_x must be 16-byte aligned. */
 int openmini_qmm_gemv_multi(const openmini_qweight_t* const* weights, int count, const float* d_x,
                             float* const* d_ys, int64_t batch, void* stream);
 
 /* FFN hidden state of FFNWeights::forward (model.rs:728-731, the silu(gate) * up
  * branch; silu(v) = v / (1 + exp(-v)), model.rs:1187-1189):
  * d_h[batch, N] = silu(x . Wg^T) * (x . Wu^T), gate and up of one type and shape, one
- * launch reading both weights for up to 3 batch rows (per 16 rows from 4 rows on).  d_x
- * must be 16-byte aligned. */
+ * launch reading both weights for up to 3 batch rows, from 4 rows on one per 16 rows or, on
+ * weights of at most 8192 rows, per 64.  d_x must be 16-byte aligned. */
 int openmini_qmm_ffn_gate_up(const openmini_qweight_t* gate, const openmini_qweight_t* up,
                              const float* d_x, float* d_h, int64_t batch, void* stream);
 

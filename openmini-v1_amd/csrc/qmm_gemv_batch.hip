@@ -611,10 +611,11 @@ struct GroupOps {
 // copied by buffer loads with an LDS destination -- whole 512-byte row spans, where
 // lanes that each load 32 bytes of their own row touch 16 lines per load -- two items
 // ahead and without registers.  LDS position p of a row holds its 16-byte segment p ^
-// (row % 8), so the reads of a lane's 8 elements are bank-conflict free.  Rows past the
+// (row % 8), which spreads the reads of a lane's 8 elements over the banks (counters: LDS
+// busy 19% of the cycles, 9% of them conflicts).  Rows past the
 // batch and elements past K read zero (out-of-range buffer offsets).
-// What bounds it: VALU issue (the split, about 150 operations per item, and 20 per tile
-// and item).  Q4_K 11008 x 4096, 40 rows: 34.8 us in three
+// What bounds it: VALU issue, 73% of the SIMDs' cycles by the counters, MFMA 18% (Q4_K 11008
+// x 4096, 40 rows; the split, about 150 operations per item, and 20 per tile and item).  Q4_K 11008 x 4096, 40 rows: 34.8 us in three
 // 16-row passes -> 22.6; 64 rows 49.7 -> 27.1; Q8_0 41.6 -> 27.5, 56.7 -> 32.0; Q4_0 4096 x
 // 4096, 64 rows 34.8 -> 17.8.
 template <int kFmt, int T, int W, int kNW, int kRH, int kMG>

@@ -120,15 +120,14 @@ inline int chunk_type(int type) { return type == OPENMINI_QMM_Q8_K ? OPENMINI_QM
 
 // The fewest activation rows from which linear() takes the fp32 GEMM on a weight of
 // n_rows x k_cols: the first m in [64, 128) where the GEMM's estimated time beats the
-// decode GEMVs', else 128.  Estimates (MI355X, graph replay): the GEMM on a grid of at
-// most one round takes about 10 ns per K element (its workgroups walk K serially:
-// K = 3072 / 4096 / 8192 / 11008 / 13824 -> 31 / 39-46 / 82-90 / 110 / 137 us at
-// 64-128 rows), a round being 512 workgroups of 64 x 64; the batched GEMV runs one
-// pass per 16 rows of about 6.5 us plus the weight bytes at 5 TB/s (Q8_0 chunks) or
-// 3 TB/s (the others).  Over 18 weight shapes x 48-112 rows (Q4_0 / Q8_0 / Q4_K /
-// Q6_K, 1024-28672 rows, K 3072-13824) the choice loses at most 9% against the faster
-// path (Q4_0 2048 x 4096 at 80 rows), a fixed 128 up to 85% (3072 x 3072 at 112 rows:
-// GEMV 60.0 vs GEMM 32.4 us).
+// decode GEMVs', else 128.  The estimates were fitted to kernels that have since become
+// faster: the GEMM on a grid of at most one round (512 workgroups of 64 x 64) at 10 ns per
+// K element, the batched GEMV at one pass per 16 rows of 6.5 us plus the weight bytes at 5
+// TB/s (Q8_0 chunks) or 3 TB/s (the others).  Measured on today's kernels (Q4_0 / Q8_0 /
+// Q4_K / Q6_K, 10 weight shapes, 33 - 127 rows) the choice is even or right on short K and
+// many rows, and up to 2.3 times the faster path on long K and few rows, which it leaves to
+// the GEMV too long: 1024 x 8192 at 96 rows GEMV 55.4, GEMM 32.1 us, 4096 x 11008 67.1
+// against 40.7; at exactly 64 rows on 10240 x 1024 it takes the GEMM 10% too early.
 inline int64_t gemm_min_rows(int type, int64_t n_rows, int64_t k_cols) {
     const double w_bytes = (double)n_rows * (double)k_cols * bytes_per_block(type) / weight_block_elems(type);
     const double pass_us = 6.5 + w_bytes / (type == OPENMINI_QMM_Q8_0 ? 5.0e6 : 3.0e6);
