@@ -747,55 +747,56 @@ int blocks_per_cu(const void* kernel, int threads) {
     return n;
 }
 
-// Shapes 0 and 7 (128 rows x 3 weight tiles per wave) are built for every instance but Q6_K on
-// bf16 x, whose super-block sums would not fit the registers.
-template <int kFmt, bool kX2>
-constexpr bool kWideTiles = kFmt != OPENMINI_QMM_Q6_K || kX2;
+// The launch shapes' rows per workgroup, column slices, K parts and weight tiles per wave, in
+// the order of choose_gemm_shape.
+constexpr int kForm[kShapes][4] = {{128, 4, 2, 3}, {128, 4, 2, 2}, {64, 2, 4, 3}, {64, 4, 2, 2},
+                                   {64, 2, 4, 2},  {64, 1, 8, 2},  {64, 2, 2, 2}, {128, 2, 2, 3}};
+// Not built for Q6_K on bf16 x: shapes 0 and 7 (the super-block sums of 128 rows x 3 weight tiles
+// would not fit the registers) and 3 (two per CU do not fit, and alone it is nowhere the fastest).
+template <int kFmt, bool kX2, int kShape>
+constexpr bool kBuilt = kFmt != OPENMINI_QMM_Q6_K || kX2 || (kShape != 0 && kShape != 3 && kShape != 7);
 
-// Workgroups per CU of the shapes' kernels (queried once per instantiation; -1: not built).
+// Workgroups per CU of a shape's kernel; -1: not built.
+template <int kFmt, bool kX2, int kShape>
+int occupancy() {
+    constexpr const int* f = kForm[kShape];
+    if constexpr (kBuilt<kFmt, kX2, kShape>)
+        return blocks_per_cu((const void*)gemm_kernel<kFmt, f[0], f[1], f[2], f[3], kX2>, 64 * f[1] * f[2]);
+    else
+        return -1;
+}
+
+// Of all shapes, queried once per instantiation.
 template <int kFmt, bool kX2>
 const int (&shape_occupancy())[kShapes] {
-    auto wide = [] {
-        if constexpr (kWideTiles<kFmt, kX2>)
-            return blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 4, 2, 3, kX2>, 512);
-        else
-            return -1;
-    };
-    auto narrow = [] {
-        if constexpr (kWideTiles<kFmt, kX2>)
-            return blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 2, 2, 3, kX2>, 256);
-        else
-            return -1;
-    };
-    static const int per_cu[kShapes] = {wide(),
-                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 128, 4, 2, 2, kX2>, 512),
-                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 4, 3, kX2>, 512),
-                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 4, 2, 2, kX2>, 512),
-                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 4, 2, kX2>, 512),
-                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 1, 8, 2, kX2>, 512),
-                                        blocks_per_cu((const void*)gemm_kernel<kFmt, 64, 2, 2, 2, kX2>, 256),
-                                        narrow()};
+    static const int per_cu[kShapes] = {occupancy<kFmt, kX2, 0>(), occupancy<kFmt, kX2, 1>(), occupancy<kFmt, kX2, 2>(),
+                                        occupancy<kFmt, kX2, 3>(), occupancy<kFmt, kX2, 4>(), occupancy<kFmt, kX2, 5>(),
+                                        occupancy<kFmt, kX2, 6>(), occupancy<kFmt, kX2, 7>()};
     return per_cu;
 }
 
 template <int kFmt, bool kX2>
 hipError_t launch_kind(const Weight& w, const uint16_t* x, const int* x_exp, float* y, int64_t m, bool gate,
                        hipStream_t s) {
+#define QMM_SHAPE_CASE(I_)                                                                                    \
+    case I_:                                                                                                  \
+        if constexpr (kBuilt<kFmt, kX2, I_>)                                                                  \
+            return launch_shape<kFmt, kForm[I_][0], kForm[I_][1], kForm[I_][2], kForm[I_][3], kX2>(           \
+                w, x, x_exp, y, m, gate, s);                                                                  \
+        break;
     switch (choose_gemm_shape(w.type, w.n_tiles, w.k, m, shape_occupancy<kFmt, kX2>(), kX2)) {
-    case 0:
-        if constexpr (kWideTiles<kFmt, kX2>) return launch_shape<kFmt, 128, 4, 2, 3, kX2>(w, x, x_exp, y, m, gate, s);
-        return hipErrorInvalidValue;
-    case 1: return launch_shape<kFmt, 128, 4, 2, 2, kX2>(w, x, x_exp, y, m, gate, s);
-    case 2: return launch_shape<kFmt, 64, 2, 4, 3, kX2>(w, x, x_exp, y, m, gate, s);
-    case 3: return launch_shape<kFmt, 64, 4, 2, 2, kX2>(w, x, x_exp, y, m, gate, s);
-    case 4: return launch_shape<kFmt, 64, 2, 4, 2, kX2>(w, x, x_exp, y, m, gate, s);
-    case 5: return launch_shape<kFmt, 64, 1, 8, 2, kX2>(w, x, x_exp, y, m, gate, s);
-    case 6: return launch_shape<kFmt, 64, 2, 2, 2, kX2>(w, x, x_exp, y, m, gate, s);
-    case 7:
-        if constexpr (kWideTiles<kFmt, kX2>) return launch_shape<kFmt, 128, 2, 2, 3, kX2>(w, x, x_exp, y, m, gate, s);
-        return hipErrorInvalidValue;
-    default: return hipErrorInvalidValue;
+        QMM_SHAPE_CASE(0)
+        QMM_SHAPE_CASE(1)
+        QMM_SHAPE_CASE(2)
+        QMM_SHAPE_CASE(3)
+        QMM_SHAPE_CASE(4)
+        QMM_SHAPE_CASE(5)
+        QMM_SHAPE_CASE(6)
+        QMM_SHAPE_CASE(7)
+    default: break;
     }
+#undef QMM_SHAPE_CASE
+    return hipErrorInvalidValue;
 }
 
 template <bool kX2>

@@ -47,8 +47,8 @@ inline int choose_gemm_shape(int type, int64_t n_tiles, int64_t k, int64_t m, co
         // bf16 x: Q8_0
         {{6.4, {13.4}}, {4.1, {9.28}}, {2.6, {4.89}}, {2.8, {6.06, 10.5}},
          {1.7, {3.46}}, {1.8, {1.92}}, {1.3, {4.39, 6.35, 8.66}}, {4.6, {10.1, 14.6}}},
-        // bf16 x: Q6_K (no 128 x 192)
-        {{}, {4.1, {13.6}}, {3.1, {7.44}}, {2.2, {9.85}},
+        // bf16 x: Q6_K (0, 3 and 7 not built)
+        {{}, {4.1, {13.6}}, {3.1, {7.44}}, {},
          {2.0, {5.19}}, {2.1, {2.61}}, {1.6, {6.60, 9.45}}, {}},
         // split x: Q4_0, Q4_K
         {{5.5, {18.9}}, {4.3, {13.7}}, {2.4, {6.25}}, {1.8, {8.37, 13.9}},

@@ -93,7 +93,7 @@ using namespace qmm;
 enum { Q4_0 = 2, Q8_0 = 7, Q4_K = 12, Q6_K = 14 };
 
 // workgroups per CU: what the kernels' registers and LDS allow on gfx950
-static const int kPerCu[6][kShapes] = {{1, 1, 1, 2, 2, 1, 4, 2}, {1, 1, 1, 2, 1, 1, 3, 2}, {-1, 1, 1, 1, 1, 1, 2, -1},
+static const int kPerCu[6][kShapes] = {{1, 1, 1, 2, 2, 1, 4, 2}, {1, 1, 1, 2, 1, 1, 3, 2}, {-1, 1, 1, -1, 1, 1, 2, -1},
                                        {1, 1, 1, 2, 2, 1, 4, 2}, {1, 1, 1, 2, 2, 1, 4, 2}, {1, 1, 1, 1, 1, 1, 3, 2}};
 static int pick(int type, int n, int k, int m, bool split) {
     return choose_gemm_shape(type, (n + 15) / 16, k, m, kPerCu[(split ? 3 : 0) + (type == Q8_0 ? 1 : type == Q6_K ? 2 : 0)], split);
@@ -127,7 +127,7 @@ int main() {
                         for (int cu : {0, 1, 2, 8}) {
                             int per_cu[kShapes];
                             for (int i = 0; i < kShapes; ++i)
-                                per_cu[i] = !split && type == Q6_K && (i == 0 || i == 7) ? -1 : cu;
+                                per_cu[i] = !split && type == Q6_K && (i == 0 || i == 3 || i == 7) ? -1 : cu;
                             const int got = choose_gemm_shape(type, tiles, k, m, per_cu, split);
                             if (got < 0 || got >= kShapes || per_cu[got] < 0) {
                                 std::printf("type %d tiles %d k %d m %d: shape %d\n", type, tiles, k, m, got);
