@@ -32,6 +32,9 @@ constexpr int kShapeTiles[kShapes] = {12, 8, 6, 8, 4, 2, 4, 6};  // weight tiles
 // (Long runs.  In the first milliseconds after idle the card is slower and small tiles lose
 // more: where Q6_K on bf16 x tied in long runs, 11008 x 4096 at 512 rows 121 us in shapes 1 and
 // 6 but 141 and 154 after idle, shape 6's row is priced 1.5% up.)
+// Left: a launch that fills its CUs exactly once with two or more workgroups each takes up to
+// 13% longer on split x than the model says (part-filled ones are right, and with weights from
+// HBM the pick still wins): 16306 x 2816 at 109 rows 35.9 us in shape 4, 32.8 in shape 3.
 struct ShapeCost {
     double start = 0.0;                 // us of a round
     double per_k[4] = {0., 0., 0., 0.}; // us of a round per 1000 K elements, 1 .. 4 workgroups on a CU
@@ -51,7 +54,7 @@ inline int choose_gemm_shape(int type, int64_t n_tiles, int64_t k, int64_t m, co
         {{}, {4.1, {13.6}}, {3.1, {7.44}}, {},
          {2.0, {5.19}}, {2.1, {2.61}}, {1.6, {6.60, 9.45}}, {}},
         // split x: Q4_0, Q4_K
-        {{5.5, {18.9}}, {4.3, {13.7}}, {2.4, {6.25}}, {1.8, {8.37, 13.9}},
+        {{6.5, {18.9}}, {4.3, {13.7}}, {2.4, {6.25}}, {1.8, {8.37, 13.9}},
          {0.7, {5.34, 8.31}}, {1.3, {2.99}}, {1.3, {7.07, 8.87, 12.4, 16.0}}, {4.7, {13.8, 20.9}}},
         // split x: Q8_0
         {{5.2, {20.3}}, {4.5, {14.5}}, {3.1, {7.07}}, {1.6, {9.00, 15.0}},
