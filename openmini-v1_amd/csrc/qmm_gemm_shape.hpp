@@ -21,8 +21,9 @@ constexpr int kShapeTiles[kShapes] = {12, 8, 6, 8, 4, 2, 4, 6};  // weight tiles
 // workgroups run in rounds of 256 CUs x as many as share one; a round costs a start (first
 // loads, K-part sums, stores) and a time per K element, a last round of j workgroups per CU
 // that of j.  Fitted to every shape forced at 27 weight shapes x 64 .. 2048 rows for Q4_0,
-// Q8_0, Q4_K and Q6_K each, and at larger ones: over those 3400 sizes the pick is on average
-// 0.1 - 0.3% slower than the fastest shape, at 43 of them by more than 3% and at most by 8%.
+// Q8_0, Q4_K and Q6_K each, and at larger ones: over the 3430 of the sweep the pick is on
+// average 0.1% slower than the fastest shape, at 28 of them by more than 3% and at most by 8%;
+// with weights that come from HBM 0.1%, 30 of 1740, 9%.
 // Types have rows of their own where their kernels' times differ: one row for Q4_0, Q8_0 and
 // Q4_K picked shapes up to 21% slower than the fastest for Q8_0 (fp32 x, 11008 x 2048 at 384
 // rows: 64.1 us against 53.0).  Shapes 6 and 7, four waves with two to four workgroups on a
